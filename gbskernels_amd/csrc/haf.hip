@@ -103,6 +103,7 @@ int haf_launch_multi(bool loop, int tier, const HafJob* jobs, int njobs, hipStre
       const int c = haf_nchunks(J.N / 2, 2 * m);
       nch_max = c > nch_max ? c : nch_max;
     }
+    if (J.N > HAF_PHASE_MAX_N && tree_parts(J.N) > nch_max) nch_max = tree_parts(J.N);
     const int64_t max_b = ((int64_t)1 << 26) / nch_max;
     const size_t per_inst = haf_workspace_bytes(loop, tier, J.N, 1);
     for (int64_t b0 = 0; b0 < J.B; b0 += max_b) {

@@ -1,4 +1,5 @@
-// haf_impl.hpp -- power-trace hafnian and loop hafnian on gfx950 (fp64, kappa, dd).
+// haf_impl.hpp -- power-trace hafnian and loop hafnian on gfx950 (every tier) for
+// sides N <= 12, and the launchers; N = 14..28 run the series tree (haf_tree.hpp).
 //
 // Algorithm (reference: core/hafnian.cu:41-133, core/loop_hafnian.cu:45-139,
 // cpu_ref/hafnian.py:60-129, cpu_ref/loop_hafnian.py:65-108):
@@ -28,12 +29,16 @@
 
 #include "cert.hpp"
 #include "common.hpp"
+#include "haf_tree.hpp"
 #include "kernels.hpp"
 
 namespace gbsk {
 
-constexpr int HAF_MAX_N = 28;
+constexpr int HAF_MAX_N = TREE_MAX_N;
 constexpr int HAF_MAX_PAIRS = HAF_MAX_N / 2;
+// sides up to this run the power-trace kernels (one launch per subset size, or
+// the fused small-size kernel), larger ones the series tree
+constexpr int HAF_PHASE_MAX_N = TREE_MIN_N - 2;
 
 // ------------------------------------------------------------ arithmetic policies
 struct ArF64 {
@@ -719,32 +724,13 @@ __device__ __forceinline__ void haf_subset_term(const typename Ar::E* __restrict
 // m = S/2 and writes the phase partial (and sum |term| in kappa mode, the
 // bound in certified mode).
 //   part[b * np + off_S + chunk]      chunk partial (np = haf_nparts(n))
-// Waves per SIMD the register allocator must leave room for, per fp64 phase
-// kernel: bit S / 2 of a mask asks for 2 (a wave capped at 256 registers, the
-// excess spilled) where the allocator alone would take more and run one wave
-// per SIMD. Plain and kappa share a mask; certified has its own. Chosen per
-// subset size from per-phase kernel times on MI355X (N = 16 and 24): forced
-// where it was faster (S = 20, 22: 1.3x; loop S = 18: 1.55x; certified
-// S = 14, 16 and loop S = 10 .. 14: 1.1 - 1.55x), left to the allocator where
-// the spill cost more (S = 24, loop S = 16, certified loop S = 16).
-#ifndef GBSK_HAF_OCC2_MASK
-#define GBSK_HAF_OCC2_MASK ((1u << 10) | (1u << 11))
-#endif
-#ifndef GBSK_HAF_OCC2_LOOP_MASK
-#define GBSK_HAF_OCC2_LOOP_MASK ((1u << 9) | (1u << 10) | (1u << 11))
-#endif
-#ifndef GBSK_HAF_OCC2_CERT_MASK
-#define GBSK_HAF_OCC2_CERT_MASK ((1u << 7) | (1u << 8))
-#endif
-#ifndef GBSK_HAF_OCC2_CERT_LOOP_MASK
-#define GBSK_HAF_OCC2_CERT_LOOP_MASK ((1u << 5) | (1u << 6) | (1u << 7))
-#endif
+// Waves per SIMD the register allocator must leave room for: two (a wave capped
+// at 256 registers, the excess spilled) for the certified loop phases S = 10, 12,
+// whose allocation would otherwise leave one wave per SIMD (1.1 - 1.55x faster
+// on MI355X); the other phases of N <= 12 fit two waves as they are.
 template <class Ar, bool LOOP, int S, int MODE>
 constexpr int haf_phase_min_waves() {
-  if (!std::is_same<Ar, ArF64>::value) return 1;
-  const unsigned mask = MODE == HM_CERT ? (LOOP ? (unsigned)GBSK_HAF_OCC2_CERT_LOOP_MASK : (unsigned)GBSK_HAF_OCC2_CERT_MASK)
-                                        : (LOOP ? (unsigned)GBSK_HAF_OCC2_LOOP_MASK : (unsigned)GBSK_HAF_OCC2_MASK);
-  return ((mask >> (S / 2)) & 1u) ? 2 : 1;
+  return std::is_same<Ar, ArF64>::value && LOOP && MODE == HM_CERT && S >= 10 ? 2 : 1;
 }
 
 template <class Ar, bool LOOP, int S, int MODE>
@@ -858,7 +844,7 @@ struct HafReduceJobs {
   const double* part_abs[HAF_MAX_JOBS];
   cplx* out[HAF_MAX_JOBS];
   double* aux[HAF_MAX_JOBS];
-  int n[HAF_MAX_JOBS];
+  int np[HAF_MAX_JOBS];  // partials per instance
   int b_begin[HAF_MAX_JOBS + 1];
   int njobs;
 };
@@ -876,8 +862,7 @@ __global__ __launch_bounds__(64 * HAF_REDUCE_WAVES) void haf_reduce_kernel(const
   if (t >= jobs.b_begin[jobs.njobs]) return;
   int jb = 0;
   while (jb + 1 < jobs.njobs && t >= jobs.b_begin[jb + 1]) ++jb;
-  const int n = jobs.n[jb];
-  const int np = haf_nparts(n);
+  const int np = jobs.np[jb];
   const int64_t b = t - jobs.b_begin[jb];
   const T* __restrict__ part = jobs.part[jb] + b * np;
   const double* __restrict__ part_abs = jobs.part_abs[jb] + b * np;
@@ -1403,7 +1388,7 @@ static void launch_phase(const HafJob* jobs, int njobs, typename Ar::T* const* p
   HafPhaseJobs<typename Ar::T> pj{};
   int wg = 0, maxN = 0;
   for (int j = 0; j < njobs; ++j) {
-    if (jobs[j].N / 2 < S / 2) continue;  // this size has no subsets of size S
+    if (jobs[j].N < S || jobs[j].N > HAF_PHASE_MAX_N) continue;  // no subsets of size S, or the series tree's
     const int k = pj.n++;
     pj.mats[k] = jobs[j].in;
     pj.part[k] = part[j];
@@ -1420,11 +1405,35 @@ static void launch_phase(const HafJob* jobs, int njobs, typename Ar::T* const* p
                      (size_t)maxN * maxN * sizeof(cplx), st, pj);
 }
 
+// Series tree of one bucket of side N = 2 H >= TREE_MIN_N: one workgroup per
+// instance and leading-pair pattern, partials [B][tree_parts(N)]. The line lies at
+// N = 14 because the power-trace kernels of N <= 12 are fused in one launch whose
+// values its own tests pin; at N = 14 (B = 4000) the tree took 249 us where the
+// per-size launches took 552 (loop 317 / 639, certified 492 / 851, dd B = 512
+// 327 / 741), at N = 24 (B = 256) 1.40 ms for 4.02, and it leads at every larger side.
+template <class Ar, bool LOOP, int MODE, int H>
+static void launch_tree_h(const HafJob& j, typename Ar::T* part, double* part_abs, hipStream_t st) {
+  const dim3 grid((unsigned)j.B * (unsigned)tree_parts(2 * H)), wg(64);
+  if constexpr (std::is_same<Ar, ArDD>::value) {
+    hipLaunchKernelGGL((haf_tree_dd_kernel<LOOP, H, MODE == HM_DDCERT>), grid, wg, 0, st, j.in, part, part_abs);
+  } else {
+    constexpr int TM = MODE == HM_KAPPA ? TM_KAPPA : (MODE == HM_CERT ? TM_CERT : TM_PLAIN);
+    hipLaunchKernelGGL((haf_tree_kernel<LOOP, H, TM>), grid, wg, 0, st, j.in, part, part_abs);
+  }
+}
+template <class Ar, bool LOOP, int MODE, int... Hs>
+static void launch_tree(const HafJob& j, typename Ar::T* part, double* part_abs, hipStream_t st,
+                        std::integer_sequence<int, Hs...>) {
+  ((j.N == 2 * Hs + TREE_MIN_N ? (launch_tree_h<Ar, LOOP, MODE, Hs + TREE_MIN_N / 2>(j, part, part_abs, st), 0) : 0),
+   ...);
+}
+
 template <class Ar, bool LOOP, int MODE, int... Ss>
 static void launch_phases(const HafJob* jobs, int njobs, typename Ar::T* const* part, double* const* part_abs,
                           hipStream_t st, std::integer_sequence<int, Ss...>) {
   int maxn = 0;
-  for (int j = 0; j < njobs; ++j) maxn = jobs[j].N / 2 > maxn ? jobs[j].N / 2 : maxn;
+  for (int j = 0; j < njobs; ++j)
+    if (jobs[j].N <= HAF_PHASE_MAX_N) maxn = jobs[j].N / 2 > maxn ? jobs[j].N / 2 : maxn;
   ((Ss + 1 <= maxn ? (launch_phase<Ar, LOOP, MODE, 2 * (Ss + 1)>(jobs, njobs, part, part_abs, st), 0) : 0), ...);
 }
 
@@ -1460,13 +1469,18 @@ int run_haf_multi(const HafJob* all, int nall, hipStream_t st) {
     rj.part_abs[j] = part_abs[j];
     rj.out[j] = jobs[j].out;
     rj.aux[j] = jobs[j].aux;
-    rj.n[j] = jobs[j].N / 2;
+    rj.np[j] = jobs[j].N > HAF_PHASE_MAX_N ? tree_parts(jobs[j].N) : haf_nparts(jobs[j].N / 2);
     rj.b_begin[j] = bsum;
     bsum += jobs[j].B;
   }
   rj.njobs = njobs;
   rj.b_begin[njobs] = bsum;
-  launch_phases<Ar, LOOP, MODE>(jobs, njobs, part, part_abs, st, std::make_integer_sequence<int, HAF_MAX_PAIRS>{});
+  launch_phases<Ar, LOOP, MODE>(jobs, njobs, part, part_abs, st,
+                                std::make_integer_sequence<int, HAF_PHASE_MAX_N / 2>{});
+  for (int j = 0; j < njobs; ++j)
+    if (jobs[j].N > HAF_PHASE_MAX_N)
+      launch_tree<Ar, LOOP, MODE>(jobs[j], part[j], part_abs[j], st,
+                                  std::make_integer_sequence<int, (TREE_MAX_N - TREE_MIN_N) / 2 + 1>{});
   hipLaunchKernelGGL((haf_reduce_kernel<Ar, MODE>), dim3((bsum + HAF_REDUCE_WAVES - 1) / HAF_REDUCE_WAVES),
                      dim3(64 * HAF_REDUCE_WAVES), 0, st, rj);
   return (int)hipGetLastError();

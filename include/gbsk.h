@@ -290,7 +290,7 @@ int gbs_perm_split(int family, int n, int* lane_log2, int* workgroups);
  * says. Several instances share a workgroup: as many as keep at least
  * small_target_wgs workgroups, or, with small_target_wgs = 0 (built in), as
  * many as a cost model of the kernel's rounds and occupancy picks per bucket;
- * larger sides run one launch per subset size.
+ * larger sides up to 12 run one launch per subset size, sides 14..28 one series-tree launch.
  * Both paths give identical values and bounds. The built-in values come from measurements
  * with gbskernels_amd/autotune.py; setting them is for tuning runs and must not
  * overlap evaluations. */
