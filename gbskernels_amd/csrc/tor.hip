@@ -22,6 +22,8 @@
 //    fully unrolled prefix-Cholesky (reference algorithm) whose factor lives in
 //    VGPRs.
 // Partials: lanes -> butterfly -> one partial per workgroup -> fixed-order sum.
+// Real policies with all T2 = 6 middle modes run the kernel of tor_tree.hpp; the
+// general workgroup here serves smaller counts and the complex policy.
 #include <type_traits>
 
 #include "cert.hpp"
@@ -612,21 +614,6 @@ __device__ inline void drop_first_mode(const T* X, int Dx, T* Y) {
 template <class Ar>
 constexpr int tor_min_waves() { return std::is_same<Ar, RF64>::value ? 3 : 1; }
 
-#ifndef TOR_BFS_Q
-#define TOR_BFS_Q 1
-#endif
-
-// Bits the breadth-first walk is split on (2^Q parts walked one after the
-// other, one part's include matrices held): 1 (two parts) for fp64, dd and
-// certified; four parts held less LDS still but their extra passes cost more
-// than the occupancy gained (fp64 1.1-1.2x, dd 1.2-1.3x slower at 12-20
-// modes). 0 for certified dd, whose walk spills 720 bytes per lane to scratch:
-// more of its workgroups per CU only thrashed the caches (20 modes 1.15x slower).
-template <class Ar>
-constexpr int tor_bfs_split() {
-  return std::is_same<Ar, RCDD>::value ? 0 : (std::is_same<Ar, RCERT>::value ? 1 : TOR_BFS_Q);
-}
-
 // Results a whole-wave launch of the fp64 tier writes itself when an instance
 // has one partial (T1 = 0), in place of the reduce or merge launch, whose
 // arithmetic on one partial is 0 + value (the other lanes' and the
@@ -640,6 +627,35 @@ struct TorDirect {
   int npc = 0;
   bool cert_inf = false;
 };
+
+// one workgroup's result (lane 0): the partial, or the final value where an
+// instance has one partial (TorDirect)
+template <class Ar, bool KAPPA, bool RERUN>
+__device__ __forceinline__ void tor_store(const typename Ar::T& acc, double aacc, bool off, int64_t b, unsigned p1,
+                                          int T1, typename Ar::P* __restrict__ part, double* __restrict__ part_abs,
+                                          const TorDirect& dir) {
+  const size_t np = (size_t)1 << T1;
+  const typename Ar::P pv = off ? Ar::part_nan() : Ar::part(acc);
+  if constexpr (std::is_same<typename Ar::P, cplx>::value && !Ar::CERT) {
+    if (dir.out != nullptr) {  // T1 = 0: b is the slot
+      const cplx s{0.0 + pv.re, 0.0 + pv.im};
+      dir.out[b] = s;
+      if (KAPPA) dir.aux[b] = 0.0 + (off ? NAN : aacc);
+      if (!RERUN && dir.cpart != nullptr) {
+        const cplx m = (s.re != s.re) ? cplx{NAN, NAN} : cplx{0.0, 0.0};
+        for (int i = 0; i < dir.npc; ++i) dir.cpart[b * dir.npc + i] = m;
+      }
+      if (RERUN && dir.cert_inf) dir.aux[b] = INFINITY;
+      return;
+    }
+  }
+  part[b * np + p1] = pv;
+  if constexpr (Ar::CERT) {
+    part_abs[b * np + p1] = off ? INFINITY : Ar::bound(acc);
+  } else if (KAPPA) {
+    part_abs[b * np + p1] = off ? NAN : aacc;
+  }
+}
 
 template <class Ar, int R, int T2, bool KAPPA, bool RERUN, bool BFS>
 __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int nm, int T1, int B,
@@ -771,18 +787,12 @@ __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int
     // (the level-0 matrix if none), shifted by two rows per exclude since.
     // Each level's new matrices are formed in one pass over the 64 lanes.
     // Pivots, complements and determinants are the depth-first walk's
-    // operations, so the values are identical; the leaf level is formed in the
-    // lanes' registers (lane k = leaf k = task k of the depth-first order).
-    // With all six middle modes the tree is walked in 2^Q parts split on the
-    // first Q modes (tor_bfs_split), one after the other, each filling its
-    // 2^(6-Q) lanes' leaves: only one part's include matrices (and the split
-    // path's) are held. At 11 modes below the leading ones: 3437 entries for
-    // the whole tree, 1950 at Q = 1, 1292 at Q = 2 (fp64: the LDS allowed 5
-    // workgroups per CU, the registers 12).
+    // operations, so the values are identical (lane k = leaf k = task k of the
+    // depth-first order).
     static_assert(Ar::SYM, "breadth-first walk of the symmetric policies");
-    constexpr int Q = (T2 == TOR_T2) ? tor_bfs_split<Ar>() : 0;  // split bits
+    static_assert(R == 0 && T2 < TOR_T2, "counts of 6 modes and more take tor_tree.hpp");
     constexpr int NODES = 1 << (T2 - 1);
-    __shared__ T bpiv[NODES][3];            // ra, rc, b01 of the current level's nodes (part-local index)
+    __shared__ T bpiv[NODES][3];            // ra, rc, b01 of the current level's nodes
     __shared__ T bdet[(2 << T2) - 1];        // determinants, level d node n at 2^d - 1 + n
     __shared__ int boff[NODES], bsh[NODES];  // each node's matrix offset and row shift
     __shared__ int region[TOR_T2 + 1];       // first entry of level d's formed matrices
@@ -799,29 +809,27 @@ __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int
       tij_c[e] = (unsigned char)j;
     }
     if (lane == 0) {
-      // level 0, then per level d >= 1 the include matrices one part holds:
-      // 2^(d-1-Q) of them above the split, one on the split path
+      // level 0, then the 2^(d-1) include matrices of each level d >= 1
       bdet[0] = det;
       int r = lev_size<true>(2 * base);
       region[0] = 0;
       for (int d = 1; d <= T2; ++d) {
         region[d] = r;
-        r += (d > Q ? (1 << (d - 1 - Q)) : 1) * lev_size<true>(2 * (base - d));
+        r += (1 << (d - 1)) * lev_size<true>(2 * (base - d));
       }
     }
     __syncthreads();
-    // pass 1 on the nodes n0 .. n0 + cnt - 1 of level d (part h): each node's
-    // matrix (offset, shift), pivots and its children's determinants
-    auto pivots = [&](int d, int h, int n0, int cnt) {
-      if (lane < cnt) {
-        const int n = n0 + lane;
+    // pass 1 on the 2^d nodes of level d: each node's matrix (offset, shift),
+    // pivots and its children's determinants
+    auto pivots = [&](int d) {
+      if (lane < (1 << d)) {
+        const int n = lane;
         int off = 0, sh = 2 * d;
         if (n != 0) {
           const int p = __builtin_ctz((unsigned)n);  // excludes since the last include
           const int lv = d - p;                      // level of the matrix that include formed
           const int g = n >> (p + 1);                // its parent at level lv - 1
-          const int loc = lv > Q ? g - (h << (lv - 1 - Q)) : 0;
-          off = region[lv] + loc * lev_size<true>(2 * (base - lv));
+          off = region[lv] + g * lev_size<true>(2 * (base - lv));
           sh = 2 * p;
         }
         const T* X = lev + off;
@@ -843,14 +851,13 @@ __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int
       __syncthreads();
     };
     // pass 2: the include child (the Schur complement of its two pivots) of
-    // each of the cnt nodes of pass 1, formed at region[d + 1] + node * Ly
-    // (part-local node index). The flat index (node, entry) is split without
+    // each node of pass 1, formed at region[d + 1] + node * Ly. The flat index (node, entry) is split without
     // an integer division (a float reciprocal, exact to one step below 2^24,
     // then corrected) and the entry's (row, column) comes from the shared table.
-    auto complements = [&](int d, int cnt) {
+    auto complements = [&](int d) {
       const int Ly = lev_size<true>(2 * (base - d - 1));
       T* const Y = lev + region[d + 1];
-      const int total = cnt * Ly;
+      const int total = Ly << d;
       const float rLy = 1.0f / (float)Ly;
       for (int idx = lane; idx < total; idx += 64) {
         int nu = (int)((float)idx * rLy);
@@ -871,52 +878,16 @@ __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int
       }
       __syncthreads();
     };
-    // the split path: level 0's node and its include child (level 1), once;
-    // deeper path levels l < Q each time the part's node there changes
-    if constexpr (Q >= 1) {
-      pivots(0, 0, 0, 1);
-      complements(0, 1);
-    }
     ntask = 1 << T2;
 #pragma unroll 1
-    for (int h = 0; h < (1 << Q); ++h) {
-      for (int l = 1; l < Q; ++l) {
-        if (h % (1 << (Q - l)) == 0) {
-          pivots(l, 0, h >> (Q - l), 1);
-          complements(l, 1);
-        }
-      }
-      for (int d = Q; d < T2; ++d) {
-        const int cnt = 1 << (d - Q);
-        pivots(d, h, h * cnt, cnt);
-        if (d + 1 < T2) complements(d, cnt);
-      }
-      // leaves of part h: lane k forms task k from its parent (level T2 - 1)
-      // in registers
-      const int k0 = h << (T2 - Q);
-      if (lane >= k0 && lane < k0 + (1 << (T2 - Q))) {
-        const int nu = (lane >> 1) - (k0 >> 1), sh = bsh[nu];
-        const T* X = lev + boff[nu];
-        const bool inc = lane & 1;
-        const T ra = bpiv[nu][0], rc = bpiv[nu][1], b01 = bpiv[nu][2];
-#pragma unroll
-        for (int e = 0; e < SLOT; ++e) {
-          const int i = tri_row(e) + 2 + sh, j = tri_col(e) + 2 + sh;
-          if (!inc) {
-            Mreg[e] = X[tri(i, j)];
-          } else {
-            const T li0 = Ar::mul(X[tri(i, sh)], ra);
-            const T li1 = Ar::mul(Ar::fms(li0, b01, X[tri(i, sh + 1)]), rc);
-            const T x0j = X[tri(j, sh)];
-            const T x1j = Ar::fms(Ar::mul(x0j, ra), b01, X[tri(j, sh + 1)]);
-            T v = Ar::fms(li0, x0j, X[tri(i, j)]);
-            Mreg[e] = Ar::fms(li1, x1j, v);
-          }
-        }
-        my_det = bdet[(1 << T2) - 1 + lane];
-        my_cnt = count + __popc((unsigned)lane);
-      }
-      __syncthreads();  // the next part overwrites the matrices above the split
+    for (int d = 0; d < T2; ++d) {
+      pivots(d);
+      if (d + 1 < T2) complements(d);
+    }
+    // no trailing modes below T2: a leaf is its determinant
+    if (lane < ntask) {
+      my_det = bdet[(1 << T2) - 1 + lane];
+      my_cnt = count + __popc((unsigned)lane);
     }
   } else {
     // cooperative walk over the T2 middle modes' include / exclude tree,
@@ -1041,29 +1012,7 @@ __device__ __forceinline__ void tor_workgroup(const cplx* __restrict__ mats, int
   acc = Ar::sum64(acc);
   if (KAPPA) aacc = group_sum<64>(aacc);
   __syncthreads();
-  if (lane == 0) {
-    const size_t np = (size_t)1 << T1;
-    const typename Ar::P pv = bad_flag ? Ar::part_nan() : Ar::part(acc);
-    if constexpr (std::is_same<typename Ar::P, cplx>::value && !Ar::CERT) {
-      if (dir.out != nullptr) {  // T1 = 0: b is the slot
-        const cplx s{0.0 + pv.re, 0.0 + pv.im};
-        dir.out[b] = s;
-        if (KAPPA) dir.aux[b] = 0.0 + (bad_flag ? NAN : aacc);
-        if (!RERUN && dir.cpart != nullptr) {
-          const cplx m = (s.re != s.re) ? cplx{NAN, NAN} : cplx{0.0, 0.0};
-          for (int i = 0; i < dir.npc; ++i) dir.cpart[b * dir.npc + i] = m;
-        }
-        if (RERUN && dir.cert_inf) dir.aux[b] = INFINITY;
-        return;
-      }
-    }
-    part[b * np + p1] = pv;
-    if constexpr (Ar::CERT) {
-      part_abs[b * np + p1] = bad_flag ? INFINITY : Ar::bound(acc);
-    } else if (KAPPA) {
-      part_abs[b * np + p1] = bad_flag ? NAN : aacc;
-    }
-  }
+  if (lane == 0) tor_store<Ar, KAPPA, RERUN>(acc, aacc, bad_flag != 0, b, p1, T1, part, part_abs, dir);
 }
 
 // RERUN: min(slots, TOR_RERUN_GRID) workgroups, each owning a contiguous range
@@ -1102,6 +1051,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tor_min_wave
     tor_workgroup<Ar, R, T2, KAPPA, RERUN, BFS>(mats, nm, T1, B, part, part_abs, blockIdx.x, dir);
   }
 }
+
+}  // namespace gbsk
+#include "tor_tree.hpp"
+namespace gbsk {
 
 // ---------------------------------------------------- small mode counts
 // When R = min(nm, RMAX) trailing modes per lane leave T2 = nm - R < 6 middle
@@ -1483,17 +1436,14 @@ __global__ void tor_n0_kernel(int B, cplx* out, double* aux, double auxval) {
   if (aux) aux[b] = auxval;
 }
 
-// LDS entries of the breadth-first walk: the level-0 matrix and, per level
-// d = 1 .. T2 - 1, the include matrices one part of the tree holds
-// (2^(d-1-Q) above the split, one on the split path; Q = tor_bfs_split at
-// T2 = TOR_T2)
-static size_t tor_bfs_entries(int nm, const TorSplit& sp, int split) {
+// LDS entries of the breadth-first walk: the level-0 matrix and the 2^(d-1)
+// include matrices of each level d = 1 .. T2 - 1
+static size_t tor_bfs_entries(int nm, const TorSplit& sp) {
   const size_t base = (size_t)(nm - sp.T1);
-  const int Q = sp.T2 == TOR_T2 ? split : 0;  // the kernel's split bits (one part held at a time)
   size_t t = base * (2 * base + 1);       // lev_size(2 base)
   for (int d = 1; d < sp.T2; ++d) {
     const size_t D = 2 * (base - d);
-    t += (d > Q ? ((size_t)1 << (d - 1 - Q)) : (size_t)1) * (D * (D + 1) / 2);
+    t += ((size_t)1 << (d - 1)) * (D * (D + 1) / 2);
   }
   return t;
 }
@@ -1506,7 +1456,7 @@ static size_t tor_lds_bytes(int nm, const TorSplit& sp, bool bfs) {
     const size_t Dd = 2 * (nm - sp.T1 - d);
     lev += Ar::SYM ? Dd * (Dd + 1) / 2 : Dd * Dd;  // the kernel's lev_size
   }
-  if (Ar::TASK_REGS && bfs) lev = tor_bfs_entries(nm, sp, tor_bfs_split<Ar>());
+  if (Ar::TASK_REGS && bfs) lev = tor_bfs_entries(nm, sp);
   const size_t slot = Ar::SYM ? (size_t)(2 * sp.R) * (2 * sp.R + 1) / 2 : (size_t)(2 * sp.R) * (2 * sp.R);
   const size_t T = sizeof(typename Ar::T);
   // task matrices in VGPRs: the level stack overlays the work matrix
@@ -1531,18 +1481,30 @@ static void launch_tor_rt1(int nm, int T1, const cplx* d_in, int B, typename Ar:
 template <class Ar, int R, int T2, bool KAPPA, bool RERUN>
 static void launch_tor_rt(int nm, int T1, const cplx* d_in, int B, typename Ar::P* part, double* part_abs, dim3 grid,
                           bool bfs, hipStream_t st, const TorDirect& dir) {
-  const TorSplit sp{R, T2, T1};
-  if constexpr (Ar::TASK_REGS && Ar::SYM && T2 >= 1) {
-    if (bfs) {
-      launch_tor_rt1<Ar, R, T2, KAPPA, RERUN, true>(nm, T1, d_in, B, part, part_abs, grid,
-                                                    tor_lds_bytes<Ar>(nm, sp, true), st, dir);
-      return;
+  if constexpr (Ar::TASK_REGS && Ar::SYM && T2 == TOR_T2) {
+    // 6 modes and more: leading modes in the lanes' registers (batched: up to
+    // TOR_BATCH_MAX_MODES modes; one large instance up to TOR_MAX_MODES, whose
+    // shorter trailing walks keep ten leading modes)
+    constexpr int LB = TOR_BATCH_MAX_MODES - TOR_T2 - Ar::RMAX, LX = TOR_MAX_MODES - TOR_T2 - R;
+    constexpr int LM = LB > 10 ? LB : 10;
+    if (T1 <= LM) {
+      hipLaunchKernelGGL((tor_tree_kernel<Ar, R, KAPPA, LM>), grid, dim3(64), 0, st, d_in, T1, part, part_abs, dir);
+    } else if constexpr (R == Ar::RMAX && !KAPPA) {
+      hipLaunchKernelGGL((tor_tree_kernel<Ar, R, KAPPA, LX>), grid, dim3(64), 0, st, d_in, T1, part, part_abs, dir);
     }
+  } else {
+    const TorSplit sp{R, T2, T1};
+    if constexpr (Ar::TASK_REGS && Ar::SYM && T2 >= 1) {
+      if (bfs) {
+        launch_tor_rt1<Ar, R, T2, KAPPA, RERUN, true>(nm, T1, d_in, B, part, part_abs, grid,
+                                                      tor_lds_bytes<Ar>(nm, sp, true), st, dir);
+        return;
+      }
+    }
+    launch_tor_rt1<Ar, R, T2, KAPPA, RERUN, false>(nm, T1, d_in, B, part, part_abs, grid,
+                                                   tor_lds_bytes<Ar>(nm, sp, false), st, dir);
   }
-  launch_tor_rt1<Ar, R, T2, KAPPA, RERUN, false>(nm, T1, d_in, B, part, part_abs, grid,
-                                                 tor_lds_bytes<Ar>(nm, sp, false), st, dir);
 }
-
 
 // the split's R and T2 are template arguments: T2 = 6 with R = 0..RMAX
 // (nm >= 6), or T2 = nm < 6 with R = 0
