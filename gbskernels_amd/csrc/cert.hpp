@@ -121,17 +121,9 @@ __device__ inline dd cdd_mul(dd a, dd b, double* e) {
 
 namespace gbsk {
 
-// r = dd_add_d(a, b); *e = |r - (a + b)|
-__device__ inline dd cdd_add_d(dd a, double b, double* e) {
-  const dd s = two_sum(a.hi, b);
-  const double w = s.lo + a.lo;
-  const dd r = fast_two_sum(s.hi, w);
-  *e = fma(CERT_U, fabs(w), cdd_fts_err(s.hi, w, r));
-  return r;
-}
 __device__ inline double cddc_norm1(ddc a) { return cdd_mag(a.re) + cdd_mag(a.im); }
-// complex dd (1-norm errors). Values are exactly ddc_add / ddc_sub / ddc_mul /
-// ddc_add_scaled of common.hpp; *e receives the operation's own error.
+// complex dd (1-norm errors). Values are exactly ddc_add / ddc_sub / ddc_mul of
+// common.hpp; *e receives the operation's own error.
 __device__ inline ddc cddc_add(ddc a, ddc b, double* e) {
   double er, ei;
   const ddc r{cdd_add(a.re, b.re, &er), cdd_add(a.im, b.im, &ei)};
@@ -139,18 +131,24 @@ __device__ inline ddc cddc_add(ddc a, ddc b, double* e) {
   return r;
 }
 __device__ inline ddc cddc_sub(ddc a, ddc b, double* e) { return cddc_add(a, ddc_neg(b), e); }
-__device__ inline ddc cddc_add_scaled(ddc a, double s, cplx z, double* e) {
-  double er, ei;
-  const ddc r{cdd_add_d(a.re, s * z.re, &er), cdd_add_d(a.im, s * z.im, &ei)};
-  *e = er + ei;
+// r = dd_mul2(a, b, c, d); *e = |r - (a b + c d)|: the six roundings of the
+// low parts, the two products of low parts, both FastTwoSums
+__device__ inline dd cdd_mul2(dd a, dd b, dd c, dd d, double* e) {
+  const dd p = two_prod(a.hi, b.hi), q = two_prod(c.hi, d.hi);
+  const double t1 = fma(a.lo, b.hi, p.lo), t = fma(a.hi, b.lo, t1);
+  const double v1 = fma(c.lo, d.hi, q.lo), v = fma(c.hi, d.lo, v1);
+  const dd h = fast_two_sum(p.hi, t), s = two_sum(h.hi, q.hi);
+  const double z = h.lo + v, w = z + s.lo;
+  const dd r = fast_two_sum(s.hi, w);
+  const double dropped = (1.0 + 2.0 * CERT_U) * (fabs(a.lo * b.lo) + fabs(c.lo * d.lo));
+  const double m = ((fabs(t1) + fabs(t)) + (fabs(v1) + fabs(v))) + (fabs(z) + fabs(w));
+  *e = fma(CERT_U, m, dropped + (cdd_fts_err(p.hi, t, h) + cdd_fts_err(s.hi, w, r)) + 8.0 * CERT_UFL);
   return r;
 }
 __device__ inline ddc cddc_mul(ddc a, ddc b, double* e) {
-  double e1, e2, e3, e4, e5, e6;
-  const dd rr = cdd_mul(a.re, b.re, &e1), ii = cdd_mul(a.im, b.im, &e2);
-  const dd ri = cdd_mul(a.re, b.im, &e3), ir = cdd_mul(a.im, b.re, &e4);
-  const ddc r{cdd_add(rr, dd_neg(ii), &e5), cdd_add(ri, ir, &e6)};
-  *e = ((e1 + e2) + (e3 + e4)) + (e5 + e6);
+  double er, ei;
+  const ddc r{cdd_mul2(a.re, b.re, dd_neg(a.im), b.im, &er), cdd_mul2(a.re, b.im, a.im, b.re, &ei)};
+  *e = er + ei;
   return r;
 }
 // bound of |a^ b^ - a b| from operand bounds ea, eb and the product's own error

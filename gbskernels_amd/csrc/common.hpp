@@ -106,15 +106,23 @@ __host__ __device__ inline ddc ddc_zero() { return ddc{dd{0.0, 0.0}, dd{0.0, 0.0
 __host__ __device__ inline ddc ddc_add(ddc a, ddc b) { return ddc{dd_add(a.re, b.re), dd_add(a.im, b.im)}; }
 __host__ __device__ inline ddc ddc_sub(ddc a, ddc b) { return ddc{dd_sub(a.re, b.re), dd_sub(a.im, b.im)}; }
 __host__ __device__ inline ddc ddc_neg(ddc a) { return ddc{dd_neg(a.re), dd_neg(a.im)}; }
+// a b + c d: both high products and the sum exact (TwoProduct, TwoSum), each
+// product's low parts in one chain, and only the first product normalised before
+// the sum: 22 operations where dd_add(dd_mul(a, b), dd_mul(c, d)) takes 27, six
+// roundings of low parts for eight; permanents by it are as far from quad values
+// (rms 0.16-0.44 x 2^-106 of sum |term| at n = 6..9, both forms). Without the first
+// normalisation 19, but the low parts' roundings grow: 8-13% further off.
+__host__ __device__ inline dd dd_mul2(dd a, dd b, dd c, dd d) {
+  const dd p = two_prod(a.hi, b.hi), q = two_prod(c.hi, d.hi);
+  const double t = fma(a.hi, b.lo, fma(a.lo, b.hi, p.lo)), v = fma(c.hi, d.lo, fma(c.lo, d.hi, q.lo));
+  const dd r = fast_two_sum(p.hi, t), s = two_sum(r.hi, q.hi);
+  return fast_two_sum(s.hi, (r.lo + v) + s.lo);
+}
 __host__ __device__ inline ddc ddc_mul(ddc a, ddc b) {
-  return ddc{dd_sub(dd_mul(a.re, b.re), dd_mul(a.im, b.im)), dd_add(dd_mul(a.re, b.im), dd_mul(a.im, b.re))};
+  return ddc{dd_mul2(a.re, b.re, dd_neg(a.im), b.im), dd_mul2(a.re, b.im, a.im, b.re)};
 }
 __host__ __device__ inline ddc ddc_mul_d(ddc a, double s) { return ddc{dd_mul_d(a.re, s), dd_mul_d(a.im, s)}; }
 __host__ __device__ inline ddc ddc_div_d(ddc a, double s) { return ddc{dd_div_d(a.re, s), dd_div_d(a.im, s)}; }
-// a + s * z with s = +-2^k (s * z exact in binary64)
-__host__ __device__ inline ddc ddc_add_scaled(ddc a, double s, cplx z) {
-  return ddc{dd_add_d(a.re, s * z.re), dd_add_d(a.im, s * z.im)};
-}
 __host__ __device__ inline cplx ddc_to_c(ddc a) { return cplx{dd_to_d(a.re), dd_to_d(a.im)}; }
 
 // |z| without spurious overflow for the kappa indicators (not on any value path)

@@ -19,6 +19,8 @@
 // partials by a fixed-order second pass. The chunking depends only on n and
 // the tier family, so a matrix's value never depends on what else is in the
 // batch.
+#include <limits.h>
+
 #include "cert.hpp"
 #include "common.hpp"
 #include "perm.hpp"
@@ -181,30 +183,81 @@ __device__ inline void glynn_range_fp64(const cplx* __restrict__ AT,  // LDS, AT
   abs_out = CERT ? E : aacc;
 }
 
+// Double-double row sums. Every entry is split once, per row and component, on
+// a grid g = 2^(k - 53) with 2^k > sum_c |a_rc|: a = hi + lo exactly, hi = g rint(a / g),
+// |lo| <= g / 2. Any sum of +-hi is a multiple of g below 2^53 g, so it is exact in
+// binary64, and a Gray step is one fma each for the high and the low sums (4 a
+// row; a double-double addition of 2a took 22 operations). The low sums round at
+// most at u |lo| <= u n g / 2, a double-double addition's own rounding, and not
+// at all where the row's entries lie within a few binary orders of one another
+// (lo is then a handful of bits). The walk hands FastTwoSum(hi, lo) to the
+// products, which is exact: hi is a multiple of ulp(lo).
+struct RowSplit {
+  int k;  // exponent; INT_MIN: nothing to split (zero, infinite or NaN row)
+  __device__ static RowSplit of(double sum) {
+    return RowSplit{sum > 0.0 && sum < INFINITY ? ilogb(fmin(sum * (1.0 + 0x1p-40), 1.79769313486231570e308)) + 1 : INT_MIN};
+  }
+  __device__ double hi(double a) const { return k == INT_MIN ? a : ldexp(rint(ldexp(a, 53 - k)), k - 53); }
+};
+
+// split the MPW staged matrices in place: AT keeps the high parts, AL gets the low
+template <int N, int MPW>
+__device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N]) {
+  for (int t = threadIdx.x; t < MPW * N * 2; t += 64) {  // (matrix, row, component)
+    const int q = t / (2 * N), r = (t >> 1) % N;
+    double* const a = reinterpret_cast<double*>(&AT[q][r]) + (t & 1);
+    double* const l = reinterpret_cast<double*>(&AL[q][r]) + (t & 1);
+    double sum = 0.0;
+#pragma unroll 4
+    for (int c = 0; c < N; ++c) sum += fabs(a[2 * c * N]);
+    const RowSplit s = RowSplit::of(sum);
+#pragma unroll 4
+    for (int c = 0; c < N; ++c) {
+      const double v = a[2 * c * N], h = s.hi(v);
+      a[2 * c * N] = h;
+      l[2 * c * N] = s.k == INT_MIN ? 0.0 : v - h;
+    }
+  }
+  __syncthreads();
+}
+
+// one row's sum as a normalised double-double
+__device__ inline ddc row_sum(cplx h, cplx l) { return ddc{fast_two_sum(h.re, l.re), fast_two_sum(h.im, l.im)}; }
+
 // Same walk in complex double-double (reference: core/permanent_dd.cu:34-73,
-// cpu_ref/permanent.py:142-189). The +-2 A entries are exact in binary64, so a
-// row-sum update is one dd + double add per component.
+// cpu_ref/permanent.py:142-189). What bounds it: FP64 issue, 842 operations
+// a term at n = 16 (16 rows at 10, 15 products at 44), 81% of the nominal rate. Measured on MI355X,
+// double-double additions and separately normalised products -> this: n = 8 / 12 /
+// 16 / 20 (B = 16384 / 16384 / 16384 / 238) 66 / 1066 / 18381 / 5501 -> 47 / 805 / 14159 /
+// 4086 us, certified n = 16 (B = 1907) 5549 -> 3139 us; values the same binary64 bits.
 template <int N>
-__device__ inline void glynn_range_dd(const cplx* __restrict__ AT, uint32_t start, int M, ddc& acc_out) {
-  ddc rs[N];
+__device__ inline void glynn_range_dd(const cplx* __restrict__ AT, const cplx* __restrict__ AL, uint32_t start, int M,
+                                      ddc& acc_out) {
+  cplx rh[N], rl[N];
   const uint32_t g = start ^ (start >> 1);
 #pragma unroll
-  for (int r = 0; r < N; ++r) rs[r] = ddc_from(AT[r]);
-#pragma unroll 1
-  for (int c = 1; c < N; ++c) {
-    const double s = ((g >> (c - 1)) & 1u) ? -1.0 : 1.0;
-#pragma unroll
-    for (int r = 0; r < N; ++r) rs[r] = ddc_add_scaled(rs[r], s, AT[c * N + r]);
+  for (int r = 0; r < N; ++r) {
+    rh[r] = AT[r];
+    rl[r] = AL[r];
   }
+  auto update = [&](double s, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      rh[r] = c_axpy(s, AT[c * N + r], rh[r]);
+      rl[r] = c_axpy(s, AL[c * N + r], rl[r]);
+    }
+  };
+#pragma unroll 1
+  for (int c = 1; c < N; ++c) update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c);
   auto product = [&]() {
     // two interleaved chains (even / odd rows), then their product
-    ddc t0 = rs[0];
+    ddc t0 = row_sum(rh[0], rl[0]);
 #pragma unroll
-    for (int r = 2; r < N; r += 2) t0 = ddc_mul(t0, rs[r]);
+    for (int r = 2; r < N; r += 2) t0 = ddc_mul(t0, row_sum(rh[r], rl[r]));
     if constexpr (N == 1) return t0;
-    ddc t1 = rs[1];
+    ddc t1 = row_sum(rh[1], rl[1]);
 #pragma unroll
-    for (int r = 3; r < N; r += 2) t1 = ddc_mul(t1, rs[r]);
+    for (int r = 3; r < N; r += 2) t1 = ddc_mul(t1, row_sum(rh[r], rl[r]));
     return ddc_mul(t0, t1);
   };
   ddc acc = product();
@@ -212,10 +265,7 @@ __device__ inline void glynn_range_dd(const cplx* __restrict__ AT, uint32_t star
   for (uint32_t j = 1; j < nsteps; ++j) {
     const int k = __builtin_ctz(j);
     const uint32_t i = start + j;
-    const double step = ((i >> (k + 1)) & 1u) ? 2.0 : -2.0;
-    const cplx* col = AT + (k + 1) * N;
-#pragma unroll
-    for (int r = 0; r < N; ++r) rs[r] = ddc_add_scaled(rs[r], step, col[r]);
+    update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     ddc p = product();
     acc = (j & 1u) ? ddc_sub(acc, p) : ddc_add(acc, p);
   }
@@ -230,39 +280,44 @@ __device__ inline void glynn_range_dd(const cplx* __restrict__ AT, uint32_t star
 __device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
 
 // glynn_range_dd with a running bound (certified double-double). The values
-// are glynn_range_dd's bit for bit. E bounds the error of every row sum (each
-// row receives the same updates, so one bound serves all rows: each step adds
-// the largest of the N update errors); products and the signed accumulation
-// propagate it with the 1-norm product rule plus each operation's own error.
+// are glynn_range_dd's bit for bit. E bounds the error of every row sum (high
+// sums are exact; each row receives the same updates, so one bound serves all
+// rows: each step adds the largest of the N low sums' roundings); products and
+// the signed accumulation propagate it with the 1-norm product rule plus each
+// operation's own error.
 template <int N>
-__device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, uint32_t start, int M, ddc& acc_out,
-                                          double& e_out) {
-  ddc rs[N];
+__device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, const cplx* __restrict__ AL, uint32_t start,
+                                          int M, ddc& acc_out, double& e_out) {
+  cplx rh[N], rl[N];
   const uint32_t g = start ^ (start >> 1);
   double E = 0.0;
 #pragma unroll
-  for (int r = 0; r < N; ++r) rs[r] = ddc_from(AT[r]);
-#pragma unroll 1
-  for (int c = 1; c < N; ++c) {
-    const double s = ((g >> (c - 1)) & 1u) ? -1.0 : 1.0;
+  for (int r = 0; r < N; ++r) {
+    rh[r] = AT[r];
+    rl[r] = AL[r];
+  }
+  auto update = [&](double s, int c) __attribute__((always_inline)) {
     double m = 0.0;
 #pragma unroll
     for (int r = 0; r < N; ++r) {
-      double e;
-      rs[r] = cddc_add_scaled(rs[r], s, AT[c * N + r], &e);
-      m = fmax(m, e);
+      rh[r] = c_axpy(s, AT[c * N + r], rh[r]);
+      rl[r] = c_axpy(s, AL[c * N + r], rl[r]);
+      m = fmax(m, cert_norm1(rl[r]));
       pin(m);
     }
-    E += m;
-  }
+    E += fma(CERT_U, m, CERT_UFL);
+  };
+#pragma unroll 1
+  for (int c = 1; c < N; ++c) update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c);
   auto product = [&](double& ep) {
-    ddc t0 = rs[0];
+    ddc t0 = row_sum(rh[0], rl[0]);
     double e0 = E;
 #pragma unroll
     for (int r = 2; r < N; r += 2) {
       double eo;
-      const ddc t = cddc_mul(t0, rs[r], &eo);
-      e0 = cddc_mul_bound(t0, e0, rs[r], E, eo);
+      const ddc rs = row_sum(rh[r], rl[r]);
+      const ddc t = cddc_mul(t0, rs, &eo);
+      e0 = cddc_mul_bound(t0, e0, rs, E, eo);
       pin(e0);
       t0 = t;
     }
@@ -270,13 +325,14 @@ __device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, uint32_t 
       ep = e0;
       return t0;
     }
-    ddc t1 = rs[1];
+    ddc t1 = row_sum(rh[1], rl[1]);
     double e1 = E;
 #pragma unroll
     for (int r = 3; r < N; r += 2) {
       double eo;
-      const ddc t = cddc_mul(t1, rs[r], &eo);
-      e1 = cddc_mul_bound(t1, e1, rs[r], E, eo);
+      const ddc rs = row_sum(rh[r], rl[r]);
+      const ddc t = cddc_mul(t1, rs, &eo);
+      e1 = cddc_mul_bound(t1, e1, rs, E, eo);
       pin(e1);
       t1 = t;
     }
@@ -291,17 +347,7 @@ __device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, uint32_t 
   for (uint32_t j = 1; j < nsteps; ++j) {
     const int k = __builtin_ctz(j);
     const uint32_t i = start + j;
-    const double step = ((i >> (k + 1)) & 1u) ? 2.0 : -2.0;
-    const cplx* col = AT + (k + 1) * N;
-    double m = 0.0;
-#pragma unroll
-    for (int r = 0; r < N; ++r) {
-      double e;
-      rs[r] = cddc_add_scaled(rs[r], step, col[r], &e);
-      m = fmax(m, e);
-      pin(m);
-    }
-    E += m;
+    update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     double ep, eo;
     const ddc p = product(ep);
     acc = (j & 1u) ? cddc_sub(acc, p, &eo) : cddc_add(acc, p, &eo);
@@ -385,13 +431,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(perm_min_wav
   const uint32_t start = ((uint32_t)chunk * LPM + (uint32_t)sub) << M;
   if constexpr (perm_is_dd(MODE)) {
     constexpr bool DDCERT = MODE == PERM_DDCERT;
+    __shared__ cplx AL[MPW][N * N];
+    split_rows<N, MPW>(AT, AL);
     ddc acc;
     double ea = 0.0;
     if constexpr (DDCERT) {
-      glynn_range_ddcert<N>(AT[gidx], start, M, acc, ea);
+      glynn_range_ddcert<N>(AT[gidx], AL[gidx], start, M, acc, ea);
       cddc_group_sum<LPM>(acc, ea);
     } else {
-      glynn_range_dd<N>(AT[gidx], start, M, acc);
+      glynn_range_dd<N>(AT[gidx], AL[gidx], start, M, acc);
       acc = group_sum<LPM>(acc);
     }
     if (sub == 0 && b < B) {
