@@ -46,11 +46,31 @@ PermSplit perm_split(int n, int family);
 int perm_lane_log2_get(int family, int n);
 int perm_lane_log2_set(int family, int n, int log2_terms);
 
+template <int... Is>
+constexpr std::integer_sequence<int, (Is + 1)...> shift1(std::integer_sequence<int, Is...>) {
+  return {};
+}
+using PermSizes = decltype(shift1(std::make_integer_sequence<int, PERM_MAX_N>{}));  // 1 .. PERM_MAX_N
+
 // Workspace bytes the launch needs for chunk partials (0 when W == 1).
 size_t perm_workspace_bytes(int n, int mode, int B);
 // Stream-ordered launch; d_aux: kappa sum|term| (PERM_KAPPA), else unused. The
 // workspace is checked against the split the launch reads (GBSK_ERR_WORKSPACE).
 int perm_launch(int n, int mode, const cplx* d_in, int B, cplx* d_out, double* d_aux, void* ws, size_t ws_size,
                 hipStream_t st);
+
+// Several uniform buckets of one mode: fp64 and kappa in one launch (and one
+// reduction) where perm_mix.hpp carries the size, else one by one. Values are
+// perm_launch's.
+struct PermJob {
+  const cplx* in;
+  cplx* out;
+  double* aux;
+  void* ws;  // perm_workspace_bytes(n, mode, B) bytes
+  size_t ws_size;
+  int n, B;
+};
+constexpr int PERM_MAX_JOBS = 28;
+int perm_launch_multi(int mode, const PermJob* jobs, int njobs, hipStream_t st);
 
 }  // namespace gbsk

@@ -1,0 +1,6 @@
+// perm_mix_kappa.hip -- the multi-size permanent launch, kappa tier.
+#include "perm_mix_impl.hpp"
+
+namespace gbsk {
+template void perm_mix_launch<PERM_KAPPA>(const PermMix&, hipStream_t);
+}
