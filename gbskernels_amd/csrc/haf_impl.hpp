@@ -924,16 +924,8 @@ __global__ __launch_bounds__(64 * HAF_REDUCE_WAVES) void haf_reduce_kernel(const
 // and reduce kernels replayed in the same order) are therefore bit-identical
 // to the phase path, and the number of instances per workgroup only changes
 // the schedule.
-constexpr int HAF_SMALL_MAX_N = 12;
 constexpr int HAF_SMALL_MAX_PAIRS = HAF_SMALL_MAX_N / 2;
 constexpr int HAF_SMALL_MAX_T = 4;  // instances per workgroup
-// certified dd takes the fused kernel up to N = 8 only: measured at B = 4096,
-// N = 8 ran 535 -> 190 us fused, but the N <= 12 class (every phase's dd
-// bound registers in one kernel) made N = 12 1.3x slower than the phases
-constexpr int HAF_SMALL_DDCERT_MAX_N = 8;
-// the dd loop hafnian likewise stops at N = 10: at B = 4096 its N <= 12 class
-// took 1978 us at N = 12 against the phases' 1484 (N = 10: 747 against 779)
-constexpr int HAF_SMALL_LHAF_DD_MAX_N = 10;
 // terms of one instance (every nonempty subset of its pairs, 2^n - 1 <= 63)
 // and chunk partials (haf_nparts(n) <= 8 for n <= 6)
 __host__ __device__ constexpr int haf_small_terms(int pairs) { return (1 << pairs) - 1; }

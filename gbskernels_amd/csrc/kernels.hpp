@@ -43,6 +43,21 @@ int tor_single_max_modes();
 size_t tor_single_workspace_bytes(int tier, int nm);
 int tor_single_launch(int tier, int nm, const cplx* d_in, cplx* d_out, double* d_aux, void* ws, hipStream_t st);
 
+// Largest sides of the fused small-size hafnian kernel: every tier but certified
+// dd and dd loop hafnians reaches HAF_SMALL_MAX_N (haf_impl.hpp).
+constexpr int HAF_SMALL_MAX_N = 12;
+// certified dd takes the fused kernel up to N = 8 only: measured at B = 4096,
+// N = 8 ran 535 -> 190 us fused, but the N <= 12 class (every phase's dd
+// bound registers in one kernel) made N = 12 1.3x slower than the phases
+constexpr int HAF_SMALL_DDCERT_MAX_N = 8;
+// the dd loop hafnian likewise stops at N = 10: at B = 4096 its N <= 12 class
+// took 1978 us at N = 12 against the phases' 1484 (N = 10: 747 against 779)
+constexpr int HAF_SMALL_LHAF_DD_MAX_N = 10;
+constexpr int haf_fused_max(bool loop, int tier) {
+  return tier == GBSK_DD_CERTIFIED ? HAF_SMALL_DDCERT_MAX_N
+                                   : (loop && tier == GBSK_DD ? HAF_SMALL_LHAF_DD_MAX_N : HAF_SMALL_MAX_N);
+}
+
 // fused small-size hafnian kernel: sizes N <= small_max_n (0..12), instances
 // per workgroup chosen to keep at least small_target_wgs workgroups (values
 // never depend on either)
