@@ -66,7 +66,8 @@ int haf_schedule_set(int small_max_n, int small_target_wgs);
 
 // torontonian schedule knobs (family 0: fp64 / kappa / certified, 1: dd /
 // certified-dd): grouped small-count kernel up to grouped_max modes (changes
-// last bits), breadth-first middle walk up to bfs_max modes (same values)
+// last bits), breadth-first middle walk up to bfs_max modes (same values; only
+// fewer than 6 modes have both walks)
 int tor_schedule_get(int family, int* grouped_max, int* bfs_max);
 int tor_schedule_set(int family, int grouped_max, int bfs_max);
 

@@ -37,9 +37,8 @@ constexpr int TOR_BATCH_MAX_MODES = 20;  // batched entry points: dim 40
 constexpr int TOR_T2 = 6;          // cooperative middle modes (64 tasks)
 // built-in schedule (tor_tune): the grouped small-count kernel up to these mode
 // counts per family (off: the breadth-first whole-wave kernel was faster at
-// every mode count), the breadth-first middle walk up to these (every count:
-// measured on MI355X, call times fp64 nm = 6 / 8 / 12 / 16 / 20 4.3x / 3.6x /
-// 2.0x / 1.6x / 1.5x faster than depth-first, dd 1.5x-4x, certified 1.2x-3.8x)
+// every mode count), the breadth-first middle walk up to these (every count the
+// general workgroup still runs: 26 -> 9.7 us at 4 modes, B = 4096, fp64)
 constexpr int TOR_GROUPED_MAX_F64 = 0;
 constexpr int TOR_GROUPED_MAX_DD = 0;
 constexpr int TOR_BFS_MAX_F64 = 32;
@@ -607,10 +606,9 @@ __device__ inline void drop_first_mode(const T* X, int Dx, T* Y) {
 // workgroup = (instance b, leading pattern p1); out partials [B][2^T1] (T)
 // RERUN: only workgroups whose partial is NaN (a real-path breakdown or a
 // complex O) run, overwriting it (the complex fallback of the fp64 tier).
-// The fp64 policy asks for three waves per SIMD: at R = 5 that is 168 VGPRs and
-// 16 spilled (the default allocation took 186-190, two waves), measured 1.2x
-// faster at 12-20 modes; four waves helped at 12-16 modes but lost at 20, and
-// the dd policies gained nothing from a hint.
+// The fp64 policy asks for three waves per SIMD: the grouped kernel at R = 5 then
+// takes 168 VGPRs and spills 12-20 (two waves otherwise); the dd policies gained
+// nothing from a hint.
 template <class Ar>
 constexpr int tor_min_waves() { return std::is_same<Ar, RF64>::value ? 3 : 1; }
 

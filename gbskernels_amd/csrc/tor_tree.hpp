@@ -23,7 +23,7 @@
 // latency of the leading steps, index work of the middle ones). Measured on
 // MI355X, general workgroup -> this kernel, B = 4096: fp64 8 / 12 / 16 modes 33.5 /
 // 206 / 3136 -> 21.7 / 101 / 1391 us, certified 8 / 12 81 / 560 -> 41 / 294 us, dd 8 / 12
-// 135 / 1492 -> 66 / 1289 us; faster at every count from 6 to 20 modes and every
+// 135 / 1492 -> 66 / 1115 us; faster at every count from 6 to 20 modes and every
 // tier. What bounds it: FP64 issue of the trailing walk (about 1500 of the 3400
 // instructions a wave runs at 16 modes) at two waves a SIMD.
 #pragma once
@@ -102,9 +102,13 @@ __device__ __forceinline__ void lane_include(const T* N, T* Y, bool inc, bool& b
   }
 }
 
-// fp64 runs two waves per SIMD (its LDS allows 8 a CU); the wider policies one.
+// fp64 and dd run two waves per SIMD (their LDS allows 8 and 7 a CU). dd at three
+// trailing modes then spills 63 VGPRs to scratch, mostly the leading columns, and
+// is still faster than one wave with 62 AGPRs: 10 / 12 / 14 modes (B = 4096 / 4096 /
+// 3051) 280 / 1298 / 4369 -> 249 / 1115 / 3636 us. The certified policies need 512
+// registers: one wave.
 template <class Ar>
-constexpr int tor_tree_waves() { return std::is_same<Ar, RF64>::value ? 2 : 1; }
+constexpr int tor_tree_waves() { return std::is_same<Ar, RF64>::value || std::is_same<Ar, RDD>::value ? 2 : 1; }
 
 // LM: leading modes the register columns have room for.
 template <class Ar, int R, bool KAPPA, int LM>
