@@ -306,7 +306,8 @@ int gbs_haf_set_schedule(int small_max_n, int small_target_wgs);
  * kernel's, so it moves values' last bits. bfs_max_modes (0..32): up to this
  * mode count the one-instance-per-wave kernel walks its middle include/exclude
  * tree breadth-first (one pass per level), depth-first above; both give
- * identical values. The built-in schedule comes from measurements with
+ * identical values. It concerns real kernels of fewer than 6 modes: from 6 on one
+ * kernel serves both settings. The built-in schedule comes from measurements with
  * gbskernels_amd/autotune.py; setting it is for tuning runs and must not
  * overlap evaluations. */
 int gbs_tor_get_schedule(int family, int* grouped_max_modes, int* bfs_max_modes);
