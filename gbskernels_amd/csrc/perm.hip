@@ -154,14 +154,15 @@ int perm_launch_multi(int mode, const PermJob* jobs, int njobs, hipStream_t st) 
   PermMix m;
   m.count = 0;
   int64_t wgs = 0, reds = 0;
+  bool big = true;
   auto flush = [&]() {
     if (!m.count) return;
     m.wg_begin[m.count] = (unsigned)wgs;
     m.red_begin[m.count] = (unsigned)reds;
     if (mode == PERM_KAPPA)
-      perm_mix_launch<PERM_KAPPA>(m, st);
+      big ? perm_mix_launch<PERM_KAPPA, true>(m, st) : perm_mix_launch<PERM_KAPPA, false>(m, st);
     else
-      perm_mix_launch<PERM_FP64>(m, st);
+      big ? perm_mix_launch<PERM_FP64, true>(m, st) : perm_mix_launch<PERM_FP64, false>(m, st);
     m.count = 0;
     wgs = reds = 0;
   };
@@ -184,6 +185,10 @@ int perm_launch_multi(int mode, const PermJob* jobs, int njobs, hipStream_t st) 
       continue;
     }
     if (sp.W > 1 && j.ws_size < (size_t)j.B * sp.W * perm_chunk_bytes(mode)) return GBSK_ERR_WORKSPACE;
+    if (big != (j.n >= PERM_MIX_BIG)) {  // sorted by side: once
+      flush();
+      big = !big;
+    }
     const int q = m.count++;
     cplx* part = reinterpret_cast<cplx*>(j.ws);
     m.in[q] = j.in;

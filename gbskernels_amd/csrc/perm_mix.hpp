@@ -16,6 +16,10 @@ namespace gbsk {
 constexpr int PERM_MIX_LDS = 1280;  // complex numbers
 template <int N>
 constexpr bool perm_mixed() { return (64 / PermCfg<N, 0>::LPM) * N * N <= PERM_MIX_LDS; }
+// Two kernels: sides from PERM_MIX_BIG on fill 256 VGPRs and spill a few, and a
+// kernel with scratch makes its queue allocate it at its first launch (a first
+// batch of small sides 820 -> 1170 us), so the smaller sides have one of their own.
+constexpr int PERM_MIX_BIG = 14;
 
 struct PermMix {  // by value in the kernel argument block
   const cplx* in[PERM_MAX_JOBS];
@@ -30,7 +34,7 @@ struct PermMix {  // by value in the kernel argument block
   int count;
 };
 
-template <int MODE>
+template <int MODE, bool BIG>
 void perm_mix_launch(const PermMix& m, hipStream_t st);
 
 }  // namespace gbsk

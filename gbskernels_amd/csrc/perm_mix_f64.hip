@@ -2,5 +2,6 @@
 #include "perm_mix_impl.hpp"
 
 namespace gbsk {
-template void perm_mix_launch<PERM_FP64>(const PermMix&, hipStream_t);
+template void perm_mix_launch<PERM_FP64, false>(const PermMix&, hipStream_t);
+template void perm_mix_launch<PERM_FP64, true>(const PermMix&, hipStream_t);
 }

@@ -2,5 +2,6 @@
 #include "perm_mix_impl.hpp"
 
 namespace gbsk {
-template void perm_mix_launch<PERM_KAPPA>(const PermMix&, hipStream_t);
+template void perm_mix_launch<PERM_KAPPA, false>(const PermMix&, hipStream_t);
+template void perm_mix_launch<PERM_KAPPA, true>(const PermMix&, hipStream_t);
 }
