@@ -1,5 +1,5 @@
 // haf_tree.hpp -- hafnian / loop hafnian of sides N = 14..28 by a subset tree of
-// Schur complements over truncated power series (fp64, kappa, certified fp64).
+// Schur complements over truncated power series (every tier).
 //
 // The subset sum is the power-trace formula's (haf_impl.hpp): with h = N / 2,
 //   haf(A) = sum_S (-1)^(h - |S|) f(S),   f(S) = [eta^h] det(I - eta X A_S)^(-1/2)
@@ -19,9 +19,8 @@
 // subsets below it: about 7e6 complex multiply-adds at N = 24 where the
 // power-trace form takes 6.5e7. Measured on MI355X, power trace -> tree: N = 16
 // (B = 4096) 1099 -> 537 us, N = 24 (B = 256) 3895 -> 1399 us, loop kappa N = 18
-// (B = 1001) 1037 -> 488 us, loop dd N = 16 (B = 512) 1789 -> 1088 us; the error
-// against double-double, relative to sum |term|, is 0.77-1.04 of the power
-// trace's (loop: 0.62), the certified bound 0.5-1.3 of it.
+// (B = 1001) 1037 -> 488 us, loop dd N = 16 (B = 512) 1789 -> 1350 us; the error
+// relative to sum |term| is 0.6-1.0 of the power trace's (loop: 0.3-0.8; dd 0.7-1.0).
 //
 // What bounds it: FP64 issue (51-56% of the cycles, 60% of it multiply-adds) and
 // the latency between a level's steps, with the waves LDS leaves room for.
@@ -804,45 +803,83 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
 
 // ------------------------------------------------------------- double-double
 // The same tree with complex double-double series; a task's two lanes form the
-// real and the imaginary part of all its coefficients. A chain of products keeps
-// (hi, lo) unnormalised: each real product exact in (p, e), hi by TwoSum, every
-// error term in lo (12 operations a product where normalised dd takes 19).
-// R: also sums |t| + |lo|, whose u-fold covers the last two roundings.
+// real and the imaginary part of all its coefficients. A chain of real products
+// starts from the value it adds to and keeps three words: high and low words are
+// summed by TwoSum, the low words' errors in lo2 (18 operations a product; 19 take a
+// normalised product and a sum), so a product leaves three roundings at the
+// 2^-106 level, those of its cross terms and of t. With the low words summed in
+// one double (12 operations, 0.85 of the time) results were 1.2-1.8 times as far
+// from quad values as the power trace's; this is 0.55-0.96 of it (N = 14 .. 20).
+// R: r receives the chain's own error: those roundings and the product of the low
+// words, which is not formed, and at the end the rounding of w and, where |w| >
+// |h.hi|, the last FastTwoSum's (a = h.hi, b = w: fl(s - a) errs by 3 u |b|, the
+// difference from it by less than u |b|). lo2's roundings, at most u K^2 <= 1.4e-12 of
+// u (|lo| at the start + sum |t|) over K <= 112 products, are in TREE_U and begin().
+struct Chain {
+  double hi = 0.0, lo = 0.0, lo2 = 0.0;
+};
 template <bool R>
-__device__ __forceinline__ void dd_mac(dd& acc, dd x, dd y, double& r) {
-  const double p = x.hi * y.hi;
-  double e = fma(x.hi, y.hi, -p);
-  e = fma(x.hi, y.lo, e);
-  e = fma(x.lo, y.hi, e);
-  const dd s = two_sum(acc.hi, p);
+__device__ __forceinline__ dd chain_value(const Chain& a, double& r) {
+  const dd h = two_sum(a.hi, a.lo);
+  const double w = h.lo + a.lo2;
+  if constexpr (R) r = fma(fabs(w) > fabs(h.hi) ? 5.0 * CERT_U : CERT_U, fabs(w), r);
+  return fast_two_sum(h.hi, w);
+}
+__device__ __forceinline__ double chain_add(Chain& a, double p, double e) {
+  const dd s = two_sum(a.hi, p);
   const double t = s.lo + e;
-  acc.hi = s.hi;
-  acc.lo += t;
-  if constexpr (R) r += fabs(t) + fabs(acc.lo);
+  const dd z = two_sum(a.lo, t);
+  a.hi = s.hi;
+  a.lo = z.hi;
+  a.lo2 += z.lo;
+  return t;
 }
 template <bool R>
-__device__ __forceinline__ void dd_mac_d(dd& acc, double x, dd y, double& r) {  // x a plain double
+__device__ __forceinline__ void dd_mac(Chain& acc, dd x, dd y, double& r) {
+  const double p = x.hi * y.hi;
+  const double f = fma(x.hi, y.lo, fma(x.hi, y.hi, -p));
+  const double e = fma(x.lo, y.hi, f);
+  const double t = chain_add(acc, p, e);
+  if constexpr (R) r += fma(fabs(x.lo), fabs(y.lo), TREE_U * ((fabs(f) + fabs(e)) + fabs(t)));
+}
+template <bool R>
+__device__ __forceinline__ void dd_mac_d(Chain& acc, double x, dd y, double& r) {  // x a plain double
   const double p = x * y.hi;
   const double e = fma(x, y.lo, fma(x, y.hi, -p));
-  const dd s = two_sum(acc.hi, p);
-  const double t = s.lo + e;
-  acc.hi = s.hi;
-  acc.lo += t;
-  if constexpr (R) r += fabs(t) + fabs(acc.lo);
+  const double t = chain_add(acc, p, e);
+  if constexpr (R) r = fma(TREE_U, fabs(e) + fabs(t), r);
 }
-__device__ __forceinline__ dd dd_fin(dd a) { return two_sum(a.hi, a.lo); }
+struct ChainC {
+  Chain re, im;
+};
+template <bool R>
+__device__ __forceinline__ ddc chain_value(const ChainC& a, double& r) {
+  const dd re = chain_value<R>(a.re, r);
+  return ddc{re, chain_value<R>(a.im, r)};
+}
 __device__ __forceinline__ dd dd_signed(dd a, double s) { return dd{s * a.hi, s * a.lo}; }
 __device__ __forceinline__ dd swap_pair_dd(dd a) { return dd{swap_pair_d(a.hi), swap_pair_d(a.lo)}; }
 
-// Certified dd: in a chain of real products TwoSum and TwoProduct are exact; e
-// (at most 3u|xy|) takes two roundings and drops x.lo y.lo: 8 u^2 |x| |y| together;
-// the additions that form t and lo err by u |t| + u |lo|, summed as they are
-// formed. A sloppy dd addition errs by at most 8 u^2 (|a| + |b|), a product with
-// a double by 4 u^2 |ab|.
-constexpr double TREE_U2 = CERT_U * CERT_U * 1.0001;
+// dd_add / dd_mul_d of one component, the operation's own error added to e
+template <bool CERT>
+__device__ __forceinline__ dd tree_add(dd a, dd b, double& e) {
+  if constexpr (!CERT) return dd_add(a, b);
+  double o;
+  const dd r = cdd_add(a, b, &o);
+  e += o;
+  return r;
+}
+template <bool CERT>
+__device__ __forceinline__ dd tree_mul_d(dd a, double b, double& e) {
+  if constexpr (!CERT) return dd_mul_d(a, b);
+  double o;
+  const dd r = cdd_mul_d(a, b, &o);
+  e += o;
+  return r;
+}
 
 template <int PM, bool CERT, int... Ps>
-__device__ __forceinline__ void tree_row_dd(ddc& s, double& es, double& r, const cplx& c, const cplx& c2, const ddc (&x)[PM],
+__device__ __forceinline__ void tree_row_dd(ChainC& s, double& es, double& r, const cplx& c, const cplx& c2, const ddc (&x)[PM],
                                             const double (&ex)[CERT ? PM : 1], int k1, std::integer_sequence<int, Ps...>) {
   auto term = [&](const cplx& z, int u) __attribute__((always_inline)) {
     dd_mac_d<CERT>(s.re, z.re, x[u].re, r);
@@ -863,7 +900,6 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
   using L = TreeLds<LOOP, H, true>;
   using S = TreeSeries<LOOP, true>;
   constexpr int T2 = TREE_T2, KC = L::KC, KS = L::KS, N = 2 * H, T1 = H - T2, RR = L::RR, PM = L::PM;
-  constexpr double G = 8.0 * TREE_U2;  // of a product's |x| |y|
   __shared__ ddc lds[L::TOTAL];
   __shared__ double ldse[CERT ? L::TOTAL : 1];  // bounds, at the same places
   dd* const ldc = reinterpret_cast<dd*>(lds);   // components: 2 i, 2 i + 1
@@ -959,20 +995,20 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
         double yA[CERT ? PM : 1];
         if constexpr (CERT) {
 #pragma unroll
-          for (int t = 0; t < PM; ++t) yA[t] = fma(G, cddc_norm1(cur[t]), ecur[t]);
+          for (int t = 0; t < PM; ++t) yA[t] = ecur[t];
         }
 #pragma unroll
         for (int i = 0; i < T1; ++i)
           if (i < k1) {
-            ddc s = ddc_zero();
+            ChainC c;
             double es = TREE_UFL, r = 0.0;
-            tree_row_dd<PM, CERT>(s, es, r, cr[i], cr2[PM > 16 ? i : 0], cur, yA, k1, std::make_integer_sequence<int, T1>{});
-            s = ddc{dd_fin(s.re), dd_fin(s.im)};
+            tree_row_dd<PM, CERT>(c, es, r, cr[i], cr2[PM > 16 ? i : 0], cur, yA, k1, std::make_integer_sequence<int, T1>{});
+            const ddc s = chain_value<CERT>(c, r);
             halves_d(s.re.hi, nxt[2 * i].re.hi, nxt[2 * i + 1].re.hi);
             halves_d(s.re.lo, nxt[2 * i].re.lo, nxt[2 * i + 1].re.lo);
             halves_d(s.im.hi, nxt[2 * i].im.hi, nxt[2 * i + 1].im.hi);
             halves_d(s.im.lo, nxt[2 * i].im.lo, nxt[2 * i + 1].im.lo);
-            if constexpr (CERT) halves_d(fma(TREE_U, r, es), enxt[2 * i], enxt[2 * i + 1]);
+            if constexpr (CERT) halves_d(es + r, enxt[2 * i], enxt[2 * i + 1]);
           }
       }
       if (isv && hf == 0) {
@@ -983,7 +1019,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
             if constexpr (CERT) ldse[vn + t * RR + vcol] = enxt[t];
           }
       }
-      auto term = [&](ddc& s, double& es, const ddc& x, double ex, const ddc& y, double ey)
+      auto term = [&](ChainC& s, double& es, const ddc& x, double ex, const ddc& y, double ey)
                       __attribute__((always_inline)) {
         double r = 0.0;
         dd_mac<CERT>(s.re, x.re, y.re, r);
@@ -992,11 +1028,10 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
         dd_mac<CERT>(s.im, x.im, y.re, r);
         if constexpr (CERT) {
           const double Y = cddc_norm1(y);
-          es = fma(cddc_norm1(x), fma(G, Y, ey), fma(ex, Y + ey, fma(TREE_U, r, es)));
+          es = fma(cddc_norm1(x), ey, fma(ex, Y + ey, es + r));
         }
       };
-      auto fin = [](const ddc& s) -> ddc { return ddc{dd_fin(s.re), dd_fin(s.im)}; };
-      ddc pe = ddc_zero(), po = ddc_zero();
+      ChainC pe, po;
       double epe = TREE_UFL, epo = TREE_UFL;
       auto swp = [](const ddc& z) -> ddc { return ddc{swap_pair_dd(z.re), swap_pair_dd(z.im)}; };
 #pragma unroll
@@ -1013,16 +1048,16 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
         }
       if (isc && hf == 0) {
         const int o = L::PB0 + (2 * j + 1) * PM + col;
-        lds[o] = ddc_mul_d(fin(pe), 2.0);
+        lds[o] = ddc_mul_d(chain_value<CERT>(pe, epe), 2.0);
         if constexpr (CERT) ldse[o] = 2.0 * epe;
         if (2 * j + 2 < H) {
-          lds[o + PM] = fin(po);
+          lds[o + PM] = chain_value<CERT>(po, epo);
           if constexpr (CERT) ldse[o + PM] = epo;
         }
       }
       __syncthreads();
       if (mine || (LOOP && lane == S::ROOT)) {
-        ddc s1 = ddc_zero(), s2 = ddc_zero();
+        ChainC s1, s2;
         double e1 = TREE_UFL, e2 = TREE_UFL;
 #pragma unroll 1
         for (int i = 0; i < k1; ++i) {
@@ -1034,16 +1069,17 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
           term(s2, e2, u0, bound(x0), lds[z1], bound(z1));
           term(s2, e2, u1, bound(x1), lds[z0], bound(z0));
         }
+        const ddc v1 = chain_value<CERT>(s1, e1), v2 = chain_value<CERT>(s2, e2);
         if (LOOP && lane == S::ROOT) {
-          lds[L::E0 + 2 * j] = fin(s1);
-          lds[L::E0 + 2 * j + 1] = fin(s2);
+          lds[L::E0 + 2 * j] = v1;
+          lds[L::E0 + 2 * j + 1] = v2;
           if constexpr (CERT) {
             ldse[L::E0 + 2 * j] = e1;
             ldse[L::E0 + 2 * j + 1] = e2;
           }
         } else {
-          put(2 * j + 1, fin(s1), e1);
-          put(2 * j + 2, fin(s2), e2);
+          put(2 * j + 1, v1, e1);
+          put(2 * j + 2, v2, e2);
         }
       }
       __syncthreads();
@@ -1060,8 +1096,8 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       ddc s = ddc_zero();
       double e = TREE_UFL;
       auto add = [&](const ddc& x, double ex) __attribute__((always_inline)) {
-        if constexpr (CERT) e = fma(8.0 * TREE_U2, cddc_norm1(s) + cddc_norm1(x), e + ex);
-        s = ddc_add(s, x);
+        e += ex;
+        s = ddc{tree_add<CERT>(s.re, x.re, e), tree_add<CERT>(s.im, x.im, e)};
       };
       if (lane == 0) {
         for (unsigned rest = p1; rest; rest &= rest - 1) {
@@ -1077,7 +1113,9 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       if constexpr (LOOP) {
         const double f = 0.5 * (lane + 1);
         const ddc x = lds[L::E0 + lane];
-        add(ddc_mul_d(x, f), CERT ? f * fma(8.0 * TREE_U2, cddc_norm1(x), bound(L::E0 + lane)) : 0.0);
+        double ex = f * bound(L::E0 + lane);
+        const ddc y{tree_mul_d<CERT>(x.re, f, ex), tree_mul_d<CERT>(x.im, f, ex)};
+        add(y, ex);
       }
       lds[L::S0 + lane] = s;
       if constexpr (CERT) ldse[L::S0 + lane] = e;
@@ -1093,7 +1131,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
   // LATE: without its product x_0 y_(d+1)); the bounds' share in e0, e1, the
   // roundings' in r0, r1. The next operands load while the present ones are used.
   struct Acc {
-    dd v{0.0, 0.0};
+    Chain v;
     double e = TREE_UFL, r = 0.0;
   };
   auto conv = [&](auto two_, auto late_, int xo, int yo, int d, double sx, Acc& a0, Acc& a1)
@@ -1106,7 +1144,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       p1v = ldc[2 * (yo + d + 1) + 1 - half];
       if constexpr (CERT) {
         const double Y = cdd_mag(p0) + cdd_mag(p1v), ey = ldse[yo + d + 1];
-        yp = fma(G, Y, ey);
+        yp = ey;
         yq = Y + ey;
       }
     }
@@ -1132,7 +1170,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       if constexpr (CERT) {
         const double X = cdd_mag(xr) + cdd_mag(xi), Y = cdd_mag(n0) + cdd_mag(n1);
         a1.e = fma(X, yp, fma(ex, yq, a1.e));
-        yp = fma(G, Y, ey);
+        yp = ey;
         yq = Y + ey;
         a0.e = fma(X, yp, fma(ex, yq, a0.e));
       }
@@ -1146,16 +1184,19 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  // closes a chain: its roundings in both components join the bound
+  // closes a chain: its errors in both components join the bound
   auto close = [&](Acc& a) __attribute__((always_inline)) -> dd {
-    if constexpr (CERT) a.e = fma(TREE_U, a.r + swap_pair_d(a.r), a.e);
-    return dd_fin(a.v);
+    const dd v = chain_value<CERT>(a.v, a.r);
+    if constexpr (CERT) a.e += a.r + swap_pair_d(a.r);
+    return v;
   };
-  // |z| of a complex value whose components lie in the two lanes of a pair
-  auto norm2 = [&](dd a) -> double {
-    const double m = cdd_mag(a);
-    return m + swap_pair_d(m);
+  auto begin = [](Acc& a, dd v) __attribute__((always_inline)) {
+    a.v.hi = v.hi;
+    a.v.lo = v.lo;
+    if constexpr (CERT) a.r = 1e-11 * CERT_U * fabs(v.lo);
   };
+  // e + the errors of both components' operations since r was zero
+  auto both = [&](double e, double r) -> double { return CERT ? e + (r + swap_pair_d(r)) : 0.0; };
 #pragma unroll 1
   for (int l = 0; l < T2; ++l) {
     const TreeTask k = tree_table<LOOP, true>.t[l][lane & ~1], kb = tree_table<LOOP, true>.t[l][lane | 1];
@@ -1165,30 +1206,37 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
     if (on) {
       const double m = isq ? -2.0 : 1.0;
       const int po = (isq ? k.px : kb.py) * KS;
-      auto rhs = [&](int d, dd s, double e) __attribute__((always_inline)) {
+      // coefficient d of m P, where its chain starts
+      auto first = [&](Acc& a, int d) __attribute__((always_inline)) {
         const int o = d < KC ? po + d : L::B0 + k.b;
-        const dd p = dd_signed(ldc[2 * o + half], m);
-        dd z = dd_add(p, s);
-        if constexpr (CERT) e = fma(8.0 * TREE_U2, norm2(p) + norm2(s), fma(fabs(m), ldse[o], e));
+        begin(a, dd_signed(ldc[2 * o + half], m));
+        if constexpr (CERT) a.e = fma(fabs(m), ldse[o], TREE_UFL);
+      };
+      auto rhs = [&](int d, dd z, double e) __attribute__((always_inline)) {
         if (isq) {
           if (d < KC) {
             ldc[2 * (k.q * KS + d) + half] = z;
             if constexpr (CERT) ldse[k.q * KS + d] = e;
           }
           const double f = -0.5 * (d + 1);
-          if constexpr (CERT) e = -f * fma(4.0 * TREE_U2, norm2(z), e);
-          z = dd_mul_d(z, f);
+          double r = 0.0;
+          z = tree_mul_d<CERT>(z, f, r);
+          e = both(-f * e, r);
         }
         if (isq || d < KC) {
           ldc[2 * (vo + d) + half] = z;
           if constexpr (CERT) ldse[vo + d] = e;
         }
       };
-      rhs(0, dd{0.0, 0.0}, TREE_UFL);
+      Acc a;
+      first(a, 0);
+      rhs(0, dd{a.v.hi, a.v.lo}, a.e);
 #pragma unroll 1
       for (int d = 0; d < H - 1; d += 2) {
         Acc a0, a1;
+        first(a0, d + 1);
         if (d + 1 < H - 1) {
+          first(a1, d + 2);
           conv(Yes{}, No{}, k.px * KS, k.py * KS, d, 1.0, a0, a1);
           conv(Yes{}, No{}, kb.px * KS, kb.py * KS, d, -1.0, a0, a1);
         } else {
@@ -1205,8 +1253,8 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
     // of the earlier ones comes through LDS)
     const int nrec = isq ? H : KC, qo = k.q * KS;
     auto start = [&](Acc& a, int o) __attribute__((always_inline)) {
-      a.v = ldc[2 * o + half];
-      if constexpr (CERT) a.e = fma(G, norm2(a.v), ldse[o]);
+      begin(a, ldc[2 * o + half]);
+      if constexpr (CERT) a.e = ldse[o];
     };
 #pragma unroll 1
     for (int d = 1; d < H; d += 2) {
@@ -1235,9 +1283,9 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
 #pragma unroll 1
       for (int d = 0; d < H; ++d) {
         const dd x = ldc[2 * (L::S0 + k.sp * H + d) + half], y = ldc[2 * (vo + d) + half];
-        ldc[2 * (vo + d) + half] = dd_add(x, y);
-        if constexpr (CERT)
-          ldse[vo + d] = fma(8.0 * TREE_U2, norm2(x) + norm2(y), bound(L::S0 + k.sp * H + d) + ldse[vo + d]);
+        double r = 0.0;
+        ldc[2 * (vo + d) + half] = tree_add<CERT>(x, y, r);
+        if constexpr (CERT) ldse[vo + d] = both(bound(L::S0 + k.sp * H + d) + ldse[vo + d], r);
       }
     }
     __syncthreads();
@@ -1248,26 +1296,34 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
         ldc[2 * (k.ed * KS) + half] = ldc[2 * (k.ez * KS) + half];
         if constexpr (CERT) ldse[k.ed * KS] = ldse[k.ez * KS];
       }
-      auto out = [&](int d, dd s, double e) __attribute__((always_inline)) {  // coefficient d of the product
+      // coefficient d of the product: a share of sigma, or added to coefficient d + 1
+      auto first = [&](Acc& a, int d) __attribute__((always_inline)) {
+        if (!isE && d + 1 < H) {
+          const int o = d + 1 < KC ? k.ez * KS + d + 1 : L::B0 + k.zb;
+          begin(a, ldc[2 * o + half]);
+          if constexpr (CERT) a.e += ldse[o];
+        }
+      };
+      auto out = [&](int d, dd s, double e) __attribute__((always_inline)) {
         if (isE) {
           const int o = L::S0 + k.esc * H + d;
           const double f = 0.5 * (d + 1);
-          const dd x = dd_mul_d(s, f), z = ldc[2 * o + half];
-          if constexpr (CERT)
-            ldse[o] = fma(8.0 * TREE_U2, norm2(x) + norm2(z), ldse[o] + f * fma(8.0 * TREE_U2, norm2(s), e));
-          ldc[2 * o + half] = dd_add(z, x);
+          double r = 0.0;
+          const dd x = tree_mul_d<CERT>(s, f, r), z = ldc[2 * o + half];
+          ldc[2 * o + half] = tree_add<CERT>(z, x, r);
+          if constexpr (CERT) ldse[o] = both(fma(f, e, ldse[o]), r);
         } else if (d + 1 < H) {
-          const int o = d + 1 < KC ? k.ez * KS + d + 1 : L::B0 + k.zb;
           const int t = d + 1 < KC ? k.ed * KS + d + 1 : L::B0 + k.db;  // TREE_BX: a slot nothing reads
-          const dd z = ldc[2 * o + half];
-          if constexpr (CERT) ldse[t] = fma(8.0 * TREE_U2, norm2(z) + norm2(s), ldse[o] + e);
-          ldc[2 * t + half] = dd_add(z, s);
+          if constexpr (CERT) ldse[t] = e;
+          ldc[2 * t + half] = s;
         }
       };
 #pragma unroll 1
       for (int d = 0; d < KC; d += 2) {
         Acc a0, a1;
+        first(a0, d);
         if (d + 1 < KC) {
+          first(a1, d + 1);
           conv(Yes{}, No{}, k.et * KS, k.ew * KS, d, 1.0, a0, a1);
           conv(Yes{}, No{}, kb.et * KS, kb.ew * KS, d, 1.0, a0, a1);
         } else {
@@ -1300,8 +1356,8 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
   for (int j = 1; j <= H; ++j) {
     if (live) {
       Acc a, none;
-      a.v = ldc[2 * (so + j - 1) + half];  // sigma_j e_0
-      if constexpr (CERT) a.e = fma(G, norm2(a.v), ldse[so + j - 1]);
+      begin(a, ldc[2 * (so + j - 1) + half]);  // sigma_j e_0
+      if constexpr (CERT) a.e += ldse[so + j - 1];
       if (j > 1) conv(No{}, No{}, so, eo, j - 2, 1.0, a, none);
       const dd s = close(a);
       const double e = a.e;
