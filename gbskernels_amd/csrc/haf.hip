@@ -40,7 +40,7 @@ __global__ void haf_trivial_kernel(int N, bool loop, int B, cplx* out, double* a
 size_t haf_workspace_bytes(bool, int tier, int N, int B) {
   if (N < 2 || (N & 1) || N > HAF_MAX_N || B <= 0) return 0;
   const size_t elem = (tier == GBSK_DD || tier == GBSK_DD_CERTIFIED) ? sizeof(ddc) : sizeof(cplx);
-  return (size_t)B * haf_nparts(N / 2) * (elem + sizeof(double));
+  return (size_t)B * haf_parts(N) * (elem + sizeof(double));
 }
 
 int haf_max_dim(bool, int tier) {

@@ -29,6 +29,7 @@
 
 #include "cert.hpp"
 #include "common.hpp"
+#include "haf_parts.hpp"
 #include "haf_tree.hpp"
 #include "kernels.hpp"
 
@@ -36,9 +37,6 @@ namespace gbsk {
 
 constexpr int HAF_MAX_N = TREE_MAX_N;
 constexpr int HAF_MAX_PAIRS = HAF_MAX_N / 2;
-// sides up to this run the power-trace kernels (one launch per subset size, or
-// the fused small-size kernel), larger ones the series tree
-constexpr int HAF_PHASE_MAX_N = TREE_MIN_N - 2;
 
 // ------------------------------------------------------------ arithmetic policies
 struct ArF64 {
@@ -242,12 +240,6 @@ __device__ inline void ddcert_group_reduce(ddc& v, double& e, ddc* red, double* 
   e = E;
 }
 
-// Work split of a phase: its C(n, m) subsets are cut into chunks of
-// HAF_CHUNK_ITERS * G consecutive subsets (G = 64 / S per wave iteration), one
-// workgroup per (instance, chunk), so that large N runs many waves per instance.
-// The split depends on (N, S) only; chunk partials are summed in chunk order.
-constexpr int HAF_CHUNK_ITERS = 1;
-__host__ __device__ inline int haf_chunk_size(int S) { return HAF_CHUNK_ITERS * (64 / S); }
 // a / b for 0 <= a < 2^16, 1 <= b <= 2^10, through one fp32 reciprocal: the
 // exact quotient (a + 1/2) / b lies at least 1/(2b) from an integer and the
 // fp32 product is within (a + 1/2) / b * 2^-21 < 2^-5 / b of it, so the
@@ -256,31 +248,6 @@ __host__ __device__ inline int haf_chunk_size(int S) { return HAF_CHUNK_ITERS * 
 __device__ __forceinline__ int small_div(int a, int b) {
   return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
 }
-__host__ __device__ constexpr int haf_cbinom(int n, int k) {
-  return (k < 0 || k > n) ? 0 : (k == 0 ? 1 : haf_cbinom(n - 1, k - 1) * n / k);
-}
-__host__ __device__ inline int haf_binom(int n, int k) {
-  if (k < 0 || k > n) return 0;
-  int r = 1;
-  for (int i = 1; i <= k; ++i) r = r * (n - k + i) / i;
-  return r;
-}
-__host__ __device__ inline int haf_nchunks(int n, int S) {
-  const int c = haf_binom(n, S / 2), ch = haf_chunk_size(S);
-  return (c + ch - 1) / ch;
-}
-// partial slots per instance (all phases) and the first slot of phase S
-__host__ __device__ inline int haf_nparts(int n) {
-  int t = 0;
-  for (int m = 1; m <= n; ++m) t += haf_nchunks(n, 2 * m);
-  return t;
-}
-__host__ __device__ inline int haf_part_offset(int n, int S) {
-  int t = 0;
-  for (int m = 1; m < S / 2; ++m) t += haf_nchunks(n, 2 * m);
-  return t;
-}
-
 // first term slot of subset size S when an instance's terms are stored size
 // by size (all C(n, 1) subsets of size 2, then the C(n, 2) of size 4, ...)
 __host__ __device__ inline int haf_small_term_offset(int n, int S) {
@@ -998,7 +965,7 @@ __device__ __forceinline__ void haf_small_phase(const typename Ar::E* As, int N,
   // chain (reads past the last subset are clamped to it and then discarded).
   // A chunk holds at most KMAX = min(G, C(PAIRS, S/2)) subsets, so only its
   // first KMAX groups are read; the idle groups after them add zero in the tail.
-  constexpr int KMAX = G < haf_cbinom(PAIRS, S / 2) ? G : haf_cbinom(PAIRS, S / 2);
+  constexpr int KMAX = G < haf_binom(PAIRS, S / 2) ? G : haf_binom(PAIRS, S / 2);
   const int nch = haf_nchunks(n, S);
   const int pbase = haf_part_offset(n, S);
   for (int idx = lane; idx < ninst * nch; idx += 64) {
@@ -1456,12 +1423,12 @@ int run_haf_multi(const HafJob* all, int nall, hipStream_t st) {
   int bsum = 0;
   for (int j = 0; j < njobs; ++j) {
     part[j] = reinterpret_cast<T*>(jobs[j].ws);
-    part_abs[j] = reinterpret_cast<double*>(part[j] + (size_t)jobs[j].B * haf_nparts(jobs[j].N / 2));
+    part_abs[j] = reinterpret_cast<double*>(part[j] + (size_t)jobs[j].B * haf_parts(jobs[j].N));
     rj.part[j] = part[j];
     rj.part_abs[j] = part_abs[j];
     rj.out[j] = jobs[j].out;
     rj.aux[j] = jobs[j].aux;
-    rj.np[j] = jobs[j].N > HAF_PHASE_MAX_N ? tree_parts(jobs[j].N) : haf_nparts(jobs[j].N / 2);
+    rj.np[j] = haf_parts(jobs[j].N);
     rj.b_begin[j] = bsum;
     bsum += jobs[j].B;
   }

@@ -35,19 +35,10 @@
 
 #include "cert.hpp"
 #include "common.hpp"
+#include "haf_parts.hpp"
 #include "kernels.hpp"
 
 namespace gbsk {
-
-constexpr int TREE_MIN_N = 14;
-constexpr int TREE_MAX_N = 28;
-// Pairs left to the tree of one workgroup (one wave); the h - 4 leading pairs'
-// include / exclude patterns are separate workgroups. A level's series tasks
-// then take up to 40 lanes (60 with the loop row) at two lanes a task, and the
-// series of a workgroup (18.9 KB at N = 24, 12.1 KB at N = 16) leave room for 8 and
-// 12 waves a CU. Five pairs with one lane a task took 54 KB at N = 24, two waves
-// a CU: 3.37 ms where this takes 1.40.
-constexpr int TREE_T2 = 4;
 
 enum TreeMode { TM_PLAIN = 0, TM_KAPPA = 1, TM_CERT = 2 };
 
@@ -61,7 +52,6 @@ __host__ __device__ constexpr int tree_region(bool loop, int lv) {
   for (int m = 1; m < lv; ++m) o += (1 << (m - 1)) * tree_size(loop, TREE_T2 - m);
   return o;
 }
-__host__ __device__ constexpr int tree_parts(int N) { return 1 << (N / 2 - TREE_T2); }
 
 // Series numbering of one workgroup's LDS: root and formed matrices, then W, then
 // q. In fp64 (DD = false) the last level's matrices overwrite W (they are formed
