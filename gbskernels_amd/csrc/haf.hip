@@ -1,6 +1,7 @@
 // haf.hip -- dispatch of the power-trace hafnian / loop hafnian launchers
 // (kernels in haf_impl.hpp, instantiated in haf_*.hip).
 #include "haf_impl.hpp"
+#include "launch_split.hpp"
 
 namespace gbsk {
 
@@ -79,9 +80,11 @@ int haf_launch_multi(bool loop, int tier, const HafJob* jobs, int njobs, hipStre
   const bool aux = tier == GBSK_KAPPA || tier == GBSK_CERTIFIED || tier == GBSK_DD_CERTIFIED;
   HafJob work[HAF_MAX_JOBS];
   int nw = 0;
+  LaunchRoom room;
   auto flush = [&]() {
     const int rc = nw ? run_multi(loop, tier, work, nw, st) : 0;
     nw = 0;
+    room = LaunchRoom{};
     return rc;
   };
   for (int j = 0; j < njobs; ++j) {
@@ -95,25 +98,20 @@ int haf_launch_multi(bool loop, int tier, const HafJob* jobs, int njobs, hipStre
       continue;
     }
     if (!J.ws) return GBSK_ERR_WORKSPACE;
-    // a job's share of one launch stays below 2^26 workgroups (at most
-    // HAF_MAX_JOBS jobs per launch: below 2^30); larger buckets are split into
-    // consecutive instance ranges, each with its own slice of the workspace
-    int nch_max = 1;
-    for (int m = 1; m <= J.N / 2; ++m) {
-      const int c = haf_nchunks(J.N / 2, 2 * m);
-      nch_max = c > nch_max ? c : nch_max;
-    }
-    if (J.N > HAF_PHASE_MAX_N && tree_parts(J.N) > nch_max) nch_max = tree_parts(J.N);
-    const int64_t max_b = ((int64_t)1 << 26) / nch_max;
+    // larger buckets are split into consecutive instance ranges, each with its own
+    // slice of the workspace (launch_split.hpp)
+    const int64_t waves = haf_launch_waves(J.N);
     const size_t per_inst = haf_workspace_bytes(loop, tier, J.N, 1);
-    for (int64_t b0 = 0; b0 < J.B; b0 += max_b) {
-      const int Bs = (int)((J.B - b0) < max_b ? (J.B - b0) : max_b);
-      if (nw == HAF_MAX_JOBS) {
+    for (int64_t b0 = 0; b0 < J.B;) {
+      const int64_t Bs = nw < HAF_MAX_JOBS ? room.take(J.B - b0, waves) : 0;
+      if (Bs == 0) {
         const int rc = flush();
         if (rc) return rc;
+        continue;
       }
       work[nw++] = HafJob{J.in + b0 * J.N * J.N, J.out + b0, aux ? J.aux + b0 : nullptr,
-                          (char*)J.ws + (size_t)b0 * per_inst, J.N, Bs};
+                          (char*)J.ws + (size_t)b0 * per_inst, J.N, (int)Bs};
+      b0 += Bs;
     }
   }
   const int rc = flush();

@@ -45,4 +45,12 @@ constexpr int haf_nparts(int n) { return haf_part_offset(n, 2 * n + 2); }
 // partials of one instance of side N (even, 2 .. TREE_MAX_N)
 constexpr int haf_parts(int N) { return N > HAF_PHASE_MAX_N ? tree_parts(N) : haf_nparts(N / 2); }
 
+// waves one instance adds to the largest of its launches (at least one: the reduction's)
+constexpr int haf_launch_waves(int N) {
+  if (N > HAF_PHASE_MAX_N) return tree_parts(N);
+  int most = 1;
+  for (int S = 2; S <= N; S += 2) most = haf_nchunks(N / 2, S) > most ? haf_nchunks(N / 2, S) : most;
+  return most;
+}
+
 }  // namespace gbsk
