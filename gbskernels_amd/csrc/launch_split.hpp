@@ -14,6 +14,14 @@ constexpr int64_t LAUNCH_WAVES = ((int64_t)1 << 26) - 4;
 // multiple of `step`
 constexpr int64_t launch_rows(int64_t waves, int64_t step = 1) { return LAUNCH_WAVES / waves / step * step; }
 
+// Workgroups of a permanent launch (one wave each): `groups` of matrices, W chunks
+// each; with W > 1 padded to a multiple of the 8 XCDs the chunks are dealt to
+// (of the groups, if fewer).
+constexpr int64_t perm_grid(int64_t groups, int W) {
+  const int64_t g8 = groups < 8 ? groups : 8;
+  return W == 1 ? groups : (groups + g8 - 1) / g8 * g8 * W;
+}
+
 // Several buckets in one launch, in order.
 struct LaunchRoom {
   int64_t used = 0;

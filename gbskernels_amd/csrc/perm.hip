@@ -2,6 +2,7 @@
 // table, one size per launch, and the multi-size launch of a batch's buckets.
 #include <algorithm>
 
+#include "launch_split.hpp"
 #include "perm_impl.hpp"
 #include "perm_mix.hpp"
 #include "perm_tune.hpp"
@@ -37,11 +38,10 @@ static int launch_perm_n(const cplx* d_in, int B, cplx* d_out, double* d_aux, vo
   const PermSplit sp = split_of<N, perm_is_dd(MODE) ? 1 : 0>();
   const int M = sp.M, W = sp.W;
   if (W > 1 && ws_size < (size_t)B * W * perm_chunk_bytes(MODE)) return GBSK_ERR_WORKSPACE;
-  // at most 2^30 workgroups per launch: large batches run as consecutive
-  // sub-batches (same stream, the workspace reused), matrices of a sub-batch a
-  // multiple of 8 groups so the XCD mapping is unchanged
-  const int64_t max_groups = (((int64_t)1 << 30) / W) / 8 * 8;
-  const int64_t max_b = max_groups * MPW;
+  // batches above the launch limit run as consecutive sub-batches (same stream,
+  // the workspace reused), matrices of a sub-batch a multiple of 8 groups so the
+  // XCD mapping is unchanged
+  const int64_t max_b = launch_rows(W, 8) * MPW;
   for (int64_t b0 = 0; b0 < B; b0 += max_b) {
     const int Bs = (int)((B - b0) < max_b ? (B - b0) : max_b);
     const cplx* in = d_in + b0 * N * N;
@@ -49,7 +49,7 @@ static int launch_perm_n(const cplx* d_in, int B, cplx* d_out, double* d_aux, vo
     double* aux = d_aux ? d_aux + b0 : nullptr;
     const int64_t groups = ((int64_t)Bs + MPW - 1) / MPW;
     const int g8 = groups < 8 ? (int)groups : 8;
-    const int64_t grid = (W == 1) ? groups : ((groups + g8 - 1) / g8) * g8 * W;
+    const int64_t grid = perm_grid(groups, W);
     if (W == 1) {
       hipLaunchKernelGGL((perm_kernel<N, MODE>), dim3((unsigned)grid), dim3(64), 0, st, in, Bs, out, aux, g8, M, W);
     } else {
@@ -178,17 +178,16 @@ int perm_launch_multi(int mode, const PermJob* jobs, int njobs, hipStream_t st) 
     const int mpw = perm_mpw(j.n);
     const int64_t groups = ((int64_t)j.B + mpw - 1) / mpw;
     const int g8 = groups < 8 ? (int)groups : 8;
-    const int64_t grid = sp.W == 1 ? groups : ((groups + g8 - 1) / g8) * g8 * sp.W;
-    if (!mix || !mixed_dispatch(j.n, PermSizes{}) || grid > (int64_t)1 << 26) {
+    const int64_t grid = perm_grid(groups, sp.W);
+    if (!mix || !mixed_dispatch(j.n, PermSizes{}) || grid > LAUNCH_WAVES) {
       const int rc = perm_launch(j.n, mode, j.in, j.B, j.out, j.aux, j.ws, j.ws_size, st);
       if (rc) return rc;
       continue;
     }
     if (sp.W > 1 && j.ws_size < (size_t)j.B * sp.W * perm_chunk_bytes(mode)) return GBSK_ERR_WORKSPACE;
-    if (big != (j.n >= PERM_MIX_BIG)) {  // sorted by side: once
-      flush();
-      big = !big;
-    }
+    const bool side = j.n >= PERM_MIX_BIG;  // sorted by side: changes once
+    if (side != big || wgs + grid > LAUNCH_WAVES) flush();
+    big = side;
     const int q = m.count++;
     cplx* part = reinterpret_cast<cplx*>(j.ws);
     m.in[q] = j.in;

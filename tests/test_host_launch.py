@@ -1,5 +1,6 @@
 """Host arithmetic of the launches (no GPU): workspace sizes, and how batches are
 cut so that every launch stays below HIP's 2^32 work-items."""
+import ctypes
 import subprocess
 from pathlib import Path
 
@@ -76,3 +77,40 @@ def test_hafnian_buckets_stay_below_the_launch_limit(tmp_path):
         assert taken == B, line
     assert all(waves[N] == 2 ** (N // 2 - 4) for N in range(14, 30, 2))
     assert waves[12] == 2 and waves[2] == 1
+
+
+PERM = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "launch_split.hpp"
+using namespace gbsk;
+int main() {
+  for (int lw = 0; lw <= 19; ++lw) {  // workgroups a matrix: 1 .. 2^19 (two terms a lane)
+    const int W = 1 << lw;
+    const long long most = launch_rows(W, 8);
+    for (long long g : {most - 1, most, most + 1})
+      std::printf("%d %lld %lld %lld\n", W, most, g, (long long)perm_grid(g, W));
+  }
+}
+"""
+
+
+def test_permanent_sub_batches_stay_below_the_launch_limit(tmp_path):
+    for line in run_split(tmp_path, PERM):
+        W, most, groups, grid = map(int, line.split())
+        assert most >= 8 and most % 8 == 0 and groups * W <= grid <= (groups + 7) * W
+        if groups <= most:
+            assert grid * 64 < 2 ** 32, line
+    # what the split gives for every size and chunking that can be set
+    k, w = ctypes.c_int(), ctypes.c_int()
+    L = _lib.lib()
+    for family in (0, 1):
+        for n in range(1, 29):
+            keep = ctypes.c_int()
+            assert L.gbs_perm_get_lane_log2(family, n, ctypes.byref(keep)) == 0
+            try:
+                assert L.gbs_perm_set_lane_log2(family, n, 2 if family else 4) == 0
+                assert L.gbs_perm_split(family, n, ctypes.byref(k), ctypes.byref(w)) == 0
+                assert w.value <= 2 ** 19
+            finally:
+                assert L.gbs_perm_set_lane_log2(family, n, keep.value) == 0
