@@ -38,6 +38,7 @@
 #include "common.hpp"
 #include "errors.hpp"
 #include "kernels.hpp"
+#include "launch_split.hpp"
 #include "sieve.hpp"
 
 namespace gbsk {
@@ -425,6 +426,21 @@ size_t sieve_partial_bytes(bool cert, int64_t parts) {
   return (size_t)parts * (sizeof(cplx) + (cert ? sizeof(double) : 0));
 }
 
+// one wave a pattern, four a workgroup (launch_split.hpp)
+static void sieve_reduce_launch(bool cert, const RepPat* d_plan, int B, const cplx* part, const double* part_e,
+                                cplx* d_out, double* d_bound, hipStream_t st) {
+  for (int64_t b0 = 0; b0 < B; b0 += LAUNCH_WAVES) {
+    const int n = (int)(B - b0 < LAUNCH_WAVES ? B - b0 : LAUNCH_WAVES);
+    const dim3 grid((unsigned)((n + 3) / 4));
+    if (cert)
+      hipLaunchKernelGGL(sieve_reduce_kernel<true>, grid, dim3(256), 0, st, d_plan + b0, n, part, part_e, d_out + b0,
+                         d_bound + b0);
+    else
+      hipLaunchKernelGGL(sieve_reduce_kernel<false>, grid, dim3(256), 0, st, d_plan + b0, n, part, part_e, d_out + b0,
+                         nullptr);
+  }
+}
+
 // d_part: sieve_partial_bytes(cert, parts) bytes; plan: host copy of d_plan
 int sieve_launch(bool cert, const cplx* d_A, const cplx* d_g, int M, const int* d_reps, int B,
                  const std::vector<RepPat>& plan, const RepPat* d_plan, int64_t parts, void* d_part, cplx* d_out,
@@ -439,13 +455,11 @@ int sieve_launch(bool cert, const cplx* d_A, const cplx* d_g, int M, const int* 
   a.part = reinterpret_cast<cplx*>(d_part);
   a.part_e = reinterpret_cast<double*>(reinterpret_cast<char*>(d_part) + (size_t)parts * sizeof(cplx));
   a.M = M;
-  // launches of at most 2^26 workgroups (64 threads each: 2^32 threads)
-  const int64_t max_wg = (int64_t)1 << 26;
   int p = 0;
   while (p < B) {
     int64_t wg = 0;
     int mm = 1, p1 = p;
-    while (p1 < B && (wg + plan[p1].chunks <= max_wg || p1 == p)) {
+    while (p1 < B && (wg + plan[p1].chunks <= LAUNCH_WAVES || p1 == p)) {
       wg += plan[p1].chunks;
       if (plan[p1].chunks) mm = std::max(mm, plan[p1].m);
       ++p1;
@@ -465,13 +479,7 @@ int sieve_launch(bool cert, const cplx* d_A, const cplx* d_g, int M, const int* 
     }
     p = p1;
   }
-  const unsigned grid = (unsigned)(((int64_t)B + 3) / 4);
-  if (cert)
-    hipLaunchKernelGGL(sieve_reduce_kernel<true>, dim3(grid), dim3(256), 0, st, d_plan, B, a.part, a.part_e, d_out,
-                       d_bound);
-  else
-    hipLaunchKernelGGL(sieve_reduce_kernel<false>, dim3(grid), dim3(256), 0, st, d_plan, B, a.part, a.part_e, d_out,
-                       d_bound);
+  sieve_reduce_launch(cert, d_plan, B, a.part, a.part_e, d_out, d_bound, st);
   return (int)hipGetLastError();
 }
 
@@ -509,13 +517,7 @@ int sieve_launch_device(bool cert, const cplx* d_A, const cplx* d_g, int M, cons
     hipLaunchKernelGGL(sieve_chunk_loop_kernel<true>, dim3(grid), dim3(64), lds, st, a, (const int64_t*)d_total);
   else
     hipLaunchKernelGGL(sieve_chunk_loop_kernel<false>, dim3(grid), dim3(64), lds, st, a, (const int64_t*)d_total);
-  const unsigned rgrid = (unsigned)(((int64_t)B + 3) / 4);
-  if (cert)
-    hipLaunchKernelGGL(sieve_reduce_kernel<true>, dim3(rgrid), dim3(256), 0, st, d_plan, B, a.part, a.part_e, d_out,
-                       d_bound);
-  else
-    hipLaunchKernelGGL(sieve_reduce_kernel<false>, dim3(rgrid), dim3(256), 0, st, d_plan, B, a.part, a.part_e, d_out,
-                       d_bound);
+  sieve_reduce_launch(cert, d_plan, B, a.part, a.part_e, d_out, d_bound, st);
   return (int)hipGetLastError();
 }
 

@@ -29,6 +29,7 @@
 #include "cert.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "launch_split.hpp"
 
 namespace gbsk {
 
@@ -1656,12 +1657,12 @@ int tor_launch(int tier, int dim, const cplx* d_in, int B, cplx* d_out, double* 
     return (int)hipGetLastError();
   }
   if (!ws) return GBSK_ERR_WORKSPACE;
-  // at most 2^30 workgroups per launch: large batches run as consecutive
-  // sub-batches on the same stream, reusing the workspace
+  // batches above the launch limit run as consecutive sub-batches on the same
+  // stream, reusing the workspace
   const TorSplit s64 = tor_batch_split<RF64>(nm), sc = tor_split(nm, RC64::RMAX), sdd = tor_batch_split<RDD>(nm);
   int t1 = s64.T1 > sc.T1 ? s64.T1 : sc.T1;
   t1 = sdd.T1 > t1 ? sdd.T1 : t1;
-  const int64_t max_b = ((int64_t)1 << 30) >> t1;
+  const int64_t max_b = launch_rows((int64_t)1 << t1);
   for (int64_t b0 = 0; b0 < B; b0 += max_b) {
     const int Bs = (int)((B - b0) < max_b ? (B - b0) : max_b);
     const cplx* in = d_in + b0 * dim * dim;

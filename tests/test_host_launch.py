@@ -114,3 +114,20 @@ def test_permanent_sub_batches_stay_below_the_launch_limit(tmp_path):
                 assert w.value <= 2 ** 19
             finally:
                 assert L.gbs_perm_set_lane_log2(family, n, keep.value) == 0
+
+
+ROWS = r"""
+#include <cstdio>
+#include "launch_split.hpp"
+int main() {
+  for (int t1 = 0; t1 <= 21; ++t1)  // workgroups an instance of the torontonian: 2^t1
+    std::printf("%d %lld\n", 1 << t1, (long long)gbsk::launch_rows((int64_t)1 << t1));
+  std::printf("4 %lld\n", (long long)gbsk::LAUNCH_WAVES / 4);  // four patterns of the sieve a workgroup
+}
+"""
+
+
+def test_rows_of_one_launch(tmp_path):
+    for line in run_split(tmp_path, ROWS):
+        waves, rows = map(int, line.split())
+        assert rows >= 1 and rows * waves * 64 < 2 ** 32 and ((rows + 3) // 4 * 256 < 2 ** 32)
