@@ -221,14 +221,42 @@ struct TreeLds {
 // TREE_UFL the underflows of a chain.
 constexpr double TREE_UFL = 1e-317;
 constexpr double TREE_U = CERT_U * 1.0000001;
-__device__ __forceinline__ double tree_rnd(cplx z, double e) { return fma(TREE_U, cert_norm1(z), e); }
-__device__ __forceinline__ double tree_im(cplx x, double ex) { return fma(TREE_U, fabs(x.im), ex); }
+__host__ __device__ __forceinline__ double tree_rnd(cplx z, double e) { return fma(TREE_U, cert_norm1(z), e); }
+__host__ __device__ __forceinline__ double tree_im(cplx x, double ex) { return fma(TREE_U, fabs(x.im), ex); }
 // one certified chain step: xs = |x| + ex, xr = ex + u |Im x| of the x operand, Y = |y|
 template <bool CERT>
-__device__ __forceinline__ void tree_mac(cplx& acc, double& e, const cplx& x, double xs, double xr, const cplx& y,
+__host__ __device__ __forceinline__ void tree_mac(cplx& acc, double& e, const cplx& x, double xs, double xr, const cplx& y,
                                          double ey, double Y) {
   if constexpr (CERT) e = fma(2.0 * TREE_U, cert_norm1(acc), fma(xs, ey, fma(xr, Y, e)));
   acc = c_fma(x, y, acc);
+}
+// acc = x y, coefficients 0 .. H - 1, one chain each: x(i, value, bound) reads x
+template <bool CERT, int H, class X>
+__host__ __device__ __forceinline__ void tree_product(const X& x, const cplx (&y)[H], const double (&ey)[CERT ? H : 1],
+                                                      cplx (&acc)[H], double (&ea)[CERT ? H : 1]) {
+  double Y[CERT ? H : 1];
+#pragma unroll
+  for (int d = 0; d < H; ++d) {
+    acc[d] = cplx{0.0, 0.0};
+    if constexpr (CERT) {
+      Y[d] = cert_norm1(y[d]);
+      ea[d] = TREE_UFL;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    cplx a;
+    double e = 0.0;
+    x(i, a, e);
+    const double xs = cert_norm1(a) + e, xr = tree_im(a, e);
+#pragma unroll
+    for (int d = i; d < H; ++d)
+      tree_mac<CERT>(acc[d], ea[CERT ? d : 0], a, xs, xr, y[d - i], ey[CERT ? d - i : 0], Y[CERT ? d - i : 0]);
+  }
+  if constexpr (CERT) {
+#pragma unroll
+    for (int d = 0; d < H; ++d) ea[d] = tree_rnd(acc[d], ea[d]);
+  }
 }
 // the bound arithmetic itself is at most this many roundings deep (cert_finish):
 // four levels of three chains, each a recurrence of depth at most 4 H^2, and
@@ -684,29 +712,13 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
         // registers) with d_0 or d_1 (half 0's y operand) and hand it over through W
         cplx acc[H];
         double ea[CERT ? H : 1];
-        if (on && !isq) {
-#pragma unroll
-          for (int d = 0; d < H; ++d) {
-            acc[d] = cplx{0.0, 0.0};
-            if constexpr (CERT) {
-              const double Y = cert_norm1(v[d]);
-              yA[d] = ev[d];
-              yB[d] = Y;
-              ea[d] = TREE_UFL;
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < H; ++i) {
-            const cplx x = lds[k.py * KS + i];
-            const double X = CERT ? cert_norm1(x) : 0.0, ex = CERT ? ldse[CERT ? k.py * KS + i : 0] : 0.0;
-#pragma unroll
-            for (int d = i; d < H; ++d) {
-              acc[d] = c_fma(x, v[d - i], acc[d]);
-              if constexpr (CERT)
-              ea[d] = fma(2.0 * TREE_U, cert_norm1(acc[d]), fma(X, yA[d - i], fma(ex, yB[d - i], ea[d])));
-            }
-          }
-        }
+        if (on && !isq)
+          tree_product<CERT, H>(
+              [&](int i, cplx& x, double& ex) __attribute__((always_inline)) {
+                x = lds[k.py * KS + i];
+                if constexpr (CERT) ex = ldse[k.py * KS + i];
+              },
+              v, ev, acc, ea);
         __syncthreads();
         if (on && !isq && !half) {
 #pragma unroll
