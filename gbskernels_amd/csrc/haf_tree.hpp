@@ -278,6 +278,20 @@ __device__ __forceinline__ void tree_row(cplx& s, double& es, const cplx& c, con
    ...);
 }
 
+// True in every lane if an entry the value depends on is not finite. The
+// elimination reads the leading rows and one triangle of the trailing block; the
+// workgroup without leading pairs, which has the least to do, looks at the rest,
+// so an entry of either triangle makes the value NaN.
+template <bool LOOP, int N>
+__device__ __forceinline__ bool tree_nonfinite(const cplx* __restrict__ A) {
+  bool bad = false;
+  for (int e = threadIdx.x; e < N * N; e += 64) {
+    const cplx z = A[e];
+    if (LOOP || e % (N + 1) != 0) bad |= !(fabs(z.re) < INFINITY && fabs(z.im) < INFINITY);
+  }
+  return __any(bad);
+}
+
 // One workgroup: instance b, include pattern p1 of the H - T2 leading pairs.
 template <bool LOOP, int H, int MODE>
 __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ mats, cplx* __restrict__ part,
@@ -328,6 +342,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
     const int r = PM + ej, i = ei < 2 * T2 ? PM + ei : r;
     put(0, (!LOOP && i == r) ? cplx{0.0, 0.0} : A[i * N + r], 0.0);
   }
+  const bool off = p1 == 0 && tree_nonfinite<LOOP, N>(A);
   if (p1 == 0) {
     if (mine) {
       for (int k = 1; k < H; ++k) put(k, cplx{0.0, 0.0}, 0.0);
@@ -798,8 +813,8 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
     coeff = group_sum<64>(coeff);
   }
   if (lane == 0) {
-    part[blockIdx.x] = coeff;
-    if constexpr (KAPPA || CERT) part_abs[blockIdx.x] = a;
+    part[blockIdx.x] = off ? cplx{NAN, NAN} : coeff;
+    if constexpr (KAPPA || CERT) part_abs[blockIdx.x] = off ? (CERT ? INFINITY : NAN) : a;
   }
 }
 
@@ -934,6 +949,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
     const int r = PM + ej, i = ei < 2 * T2 ? PM + ei : r;
     put(0, ddc_from((!LOOP && i == r) ? cplx{0.0, 0.0} : A[i * N + r]), 0.0);
   }
+  const bool off = p1 == 0 && tree_nonfinite<LOOP, N>(A);
   if (p1 == 0) {
     if (mine) {
       for (int k = 1; k < H; ++k) put(k, ddc_zero(), 0.0);
@@ -1394,9 +1410,9 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
     }
   }
   if (lane < 2) {
-    reinterpret_cast<dd*>(part)[2 * (int64_t)blockIdx.x + lane] = coeff;
+    reinterpret_cast<dd*>(part)[2 * (int64_t)blockIdx.x + lane] = off ? dd{NAN, NAN} : coeff;
     if constexpr (CERT) {
-      if (lane == 0) part_abs[blockIdx.x] = cert_finish(ecoeff, TREE_DEPTH);
+      if (lane == 0) part_abs[blockIdx.x] = off ? INFINITY : cert_finish(ecoeff, TREE_DEPTH);
     }
   }
 }
