@@ -21,6 +21,11 @@
 // (B = 4096) 1099 -> 537 us, N = 24 (B = 256) 3895 -> 1399 us, loop kappa N = 18
 // (B = 1001) 1037 -> 488 us, loop dd N = 16 (B = 512) 1789 -> 1350 us; the error
 // relative to sum |term| is 0.6-1.0 of the power trace's (loop: 0.3-0.8; dd 0.7-1.0).
+// Certified bounds, medians against the power trace's: fp64, complex matrices 0.61 /
+// 0.59 / 0.47 / 0.41 / 0.31 / 0.24 at N = 14 .. 24 (loop 0.43 .. 0.17); real ones, where the
+// tree's longer sums show, 1.08 / 1.08 / 1.04 at N = 14 / 16 / 18 (single matrices up to
+// 3.4), 0.87 and less from 20 on (loop 0.89 and less); dd 1.9 / 2.0 / 1.9 / 1.7 at N = 14 ..
+// 20 (loop 1.8 .. 1.1), real 1.8 / 2.3 / 2.5 at N = 14 / 16 / 18 (loop 2.0 / 2.1 / 2.1).
 //
 // What bounds it: FP64 issue (51-56% of the cycles, 60% of it multiply-adds) and
 // the latency between a level's steps, with the waves LDS leaves room for.
@@ -210,17 +215,26 @@ struct TreeLds {
   static_assert(PM + RR <= 32, "one column a lane of each half wave");
 };
 
-// Certified bounds (1-norm, cert.hpp): every value formed here is a chain
-// acc = c_fma(x_i, y_i, acc) plus single operations on its result. One step's
-// four roundings (common.hpp c_fma: the products with Im x go first) are at most
-//   u (|acc_before| + |Im x_i| |y_i|) + u |acc_after|   (up to the factor 1 + u),
-// |z| = |Re z| + |Im z|; so a step charges 2 u |acc_before| and
+// Certified bounds (of the modulus; model and bound arithmetic: cert.hpp): every
+// value formed here is a chain acc = c_fma(x_i, y_i, acc) plus single operations on
+// its result. One step's four roundings (common.hpp c_fma: the products with Im x
+// go first) are at most
+//   u (|acc_before| + |Im x_i| |y_i|) + u |acc_after|   (up to the factor 1 + u);
+// so a step charges 2 u |acc_before| and
 //   |x| ey + ex (|y| + ey) + u |Im x| |y| = (|x| + ex) ey + (ex + u |Im x|) |y|
 // for its operands' bounds ex, ey, the chain's end u |acc|, and each further
 // operation its own rounding u |result|. TREE_U carries the factors 1 + u,
-// TREE_UFL the underflows of a chain.
+// TREE_UFL the underflows of a chain. Roundings take |Re| + |Im| for |z|; the factors
+// of a bound take tree_abs, since products nest deeper here than in the power trace
+// and |Re| + |Im| is 1.27 |z| on average: with it bounds were 3 times as wide.
 constexpr double TREE_UFL = 1e-317;
 constexpr double TREE_U = CERT_U * 1.0000001;
+// |a + ib| from above: the chord of sqrt(1 + t^2) over t = 0 .. 1, at most 8% more. A NaN may
+// be dropped: it is in the value as well, whose own rounding then refuses the bound.
+__host__ __device__ __forceinline__ double tree_abs(double a, double b) {
+  return fma(0.41421356237309515, fmin(fabs(a), fabs(b)), fmax(fabs(a), fabs(b)));
+}
+__host__ __device__ __forceinline__ double tree_abs(cplx z) { return tree_abs(z.re, z.im); }
 __host__ __device__ __forceinline__ double tree_rnd(cplx z, double e) { return fma(TREE_U, cert_norm1(z), e); }
 __host__ __device__ __forceinline__ double tree_im(cplx x, double ex) { return fma(TREE_U, fabs(x.im), ex); }
 // one certified chain step: xs = |x| + ex, xr = ex + u |Im x| of the x operand, Y = |y|
@@ -239,7 +253,7 @@ __host__ __device__ __forceinline__ void tree_product(const X& x, const cplx (&y
   for (int d = 0; d < H; ++d) {
     acc[d] = cplx{0.0, 0.0};
     if constexpr (CERT) {
-      Y[d] = cert_norm1(y[d]);
+      Y[d] = tree_abs(y[d]);
       ea[d] = TREE_UFL;
     }
   }
@@ -248,7 +262,7 @@ __host__ __device__ __forceinline__ void tree_product(const X& x, const cplx (&y
     cplx a;
     double e = 0.0;
     x(i, a, e);
-    const double xs = cert_norm1(a) + e, xr = tree_im(a, e);
+    const double xs = tree_abs(a) + e, xr = tree_im(a, e);
 #pragma unroll
     for (int d = i; d < H; ++d)
       tree_mac<CERT>(acc[d], ea[CERT ? d : 0], a, xs, xr, y[d - i], ey[CERT ? d - i : 0], Y[CERT ? d - i : 0]);
@@ -269,7 +283,7 @@ template <int PM, bool CERT, int... Ps>
 __device__ __forceinline__ void tree_row(cplx& s, double& es, const cplx& c, const cplx& c2, const cplx (&x)[PM],
                                          const double (&ex)[CERT ? PM : 1], int k1, std::integer_sequence<int, Ps...>) {
   auto term = [&](const cplx& z, int u) __attribute__((always_inline)) {
-    if constexpr (CERT) es = fma(2.0 * TREE_U, cert_norm1(s), fma(cert_norm1(z), ex[u], es));
+    if constexpr (CERT) es = fma(2.0 * TREE_U, cert_norm1(s), fma(tree_abs(z), ex[u], es));
     s = c_fma(z, x[u], s);
   };
   (((Ps < k1) ? (term(row_bcast<(2 * Ps) % 16>(Ps < 8 ? c : c2), 2 * Ps),
@@ -432,7 +446,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
       double epe = TREE_UFL, epo = TREE_UFL;
       auto term = [&](cplx& s, double& es, const cplx& x, double ex, const cplx& y, double ey)
                       __attribute__((always_inline)) {
-        tree_mac<CERT>(s, es, x, cert_norm1(x) + ex, tree_im(x, ex), y, ey, cert_norm1(y));
+        tree_mac<CERT>(s, es, x, tree_abs(x) + ex, tree_im(x, ex), y, ey, tree_abs(y));
       };
 #pragma unroll
       for (int i = 0; i < T1; ++i)
@@ -563,7 +577,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
         y[d] = d < KC ? py[d] : bx[k.b];
         v[d] = cplx{0.0, 0.0};
         if constexpr (CERT) {
-          const double ey = d < KC ? ldse[k.py * KS + d] : bxe[k.b], Y = cert_norm1(y[d]);
+          const double ey = d < KC ? ldse[k.py * KS + d] : bxe[k.b], Y = tree_abs(y[d]);
           yA[d] = ey;
           yB[d] = Y;
           ev[d] = fma(fabs(m), ey, TREE_UFL);
@@ -573,7 +587,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
       for (int i = 0; i < H - 1; ++i) {
         const cplx x = c_scale(px[i], sg);
         const double ex = CERT ? ldse[CERT ? k.px * KS + i : 0] : 0.0;
-        const double xs = cert_norm1(x) + ex, xr = tree_im(x, ex);
+        const double xs = tree_abs(x) + ex, xr = tree_im(x, ex);
 #pragma unroll
         for (int d = i; d < H - 1; ++d)
           tree_mac<CERT>(v[d + 1], ev[CERT ? d + 1 : 0], x, xs, xr, y[d - i], yA[CERT ? d - i : 0], yB[CERT ? d - i : 0]);
@@ -605,7 +619,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
       for (int d = 0; d < H - 1; ++d) {
         y[d] = c_neg(shareq ? lds[k.q * KS + d] : v[d]);
         if constexpr (CERT) {
-          const double ey = shareq ? ldse[k.q * KS + d] : ev[d], Y = cert_norm1(y[d]);
+          const double ey = shareq ? ldse[k.q * KS + d] : ev[d], Y = tree_abs(y[d]);
           yA[d] = ey;
           yB[d] = Y;
         }
@@ -622,7 +636,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
         // v[0] is no chain
         if constexpr (CERT) ev[i - 1] = i > 1 ? tree_rnd(x, ev[i - 1]) : ev[0];
         const double ex = CERT ? ev[CERT ? i - 1 : 0] : 0.0;
-        const double xs = cert_norm1(x) + ex, xr = tree_im(x, ex);
+        const double xs = tree_abs(x) + ex, xr = tree_im(x, ex);
 #pragma unroll
         for (int d = i; d < H; ++d)
           tree_mac<CERT>(v[d], ev[CERT ? d : 0], x, xs, xr, y[d - i], yA[CERT ? d - i : 0], yB[CERT ? d - i : 0]);
@@ -664,7 +678,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
           y[d] = lds[k.ew * KS + d];
           acc[d] = cplx{0.0, 0.0};
           if constexpr (CERT) {
-            const double ey = ldse[k.ew * KS + d], Y = cert_norm1(y[d]);
+            const double ey = ldse[k.ew * KS + d], Y = tree_abs(y[d]);
             yA[d] = ey;
             yB[d] = Y;
             ea[d] = TREE_UFL;
@@ -674,7 +688,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
         for (int i = 0; i < KC; ++i) {
           const cplx x = lds[k.et * KS + i];
           const double ex = CERT ? ldse[CERT ? k.et * KS + i : 0] : 0.0;
-          const double xs = cert_norm1(x) + ex, xr = tree_im(x, ex);
+          const double xs = tree_abs(x) + ex, xr = tree_im(x, ex);
 #pragma unroll
           for (int d = i; d < KC; ++d)
             tree_mac<CERT>(acc[d], ea[CERT ? d : 0], x, xs, xr, y[d - i], yA[CERT ? d - i : 0], yB[CERT ? d - i : 0]);
@@ -768,7 +782,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
         if constexpr (CERT) {
 #pragma unroll
           for (int d = 0; d < H; ++d) {
-            const double Y = cert_norm1(v[d]);
+            const double Y = tree_abs(v[d]);
             yA[d] = ev[d];
             yB[d] = Y;
           }
@@ -785,7 +799,7 @@ __global__ __launch_bounds__(64) void haf_tree_kernel(const cplx* __restrict__ m
             e.im = fma(fma(-(double)j, e.im, s[j].im), r, e.im);
             if constexpr (CERT) ee = fma(tree_rnd(s[j], es[j]), (1.0 + 8.0 * CERT_U) / j, 4.0 * CERT_U * cert_norm1(e));
           }
-          const double xs = cert_norm1(e) + ee, xr = tree_im(e, ee);
+          const double xs = tree_abs(e) + ee, xr = tree_im(e, ee);
           if (j == H) {
             coeff = e;
             ecoeff = ee;
@@ -869,6 +883,7 @@ __device__ __forceinline__ void dd_mac_d(Chain& acc, double x, dd y, double& r) 
 struct ChainC {
   Chain re, im;
 };
+__device__ __forceinline__ double tree_abs(ddc z) { return tree_abs(cdd_mag(z.re), cdd_mag(z.im)); }
 template <bool R>
 __device__ __forceinline__ ddc chain_value(const ChainC& a, double& r) {
   const dd re = chain_value<R>(a.re, r);
@@ -903,7 +918,7 @@ __device__ __forceinline__ void tree_row_dd(ChainC& s, double& es, double& r, co
     dd_mac_d<CERT>(s.im, z.re, x[u].im, r);
     dd_mac_d<CERT>(s.re, -z.im, x[u].im, r);
     dd_mac_d<CERT>(s.im, z.im, x[u].re, r);
-    if constexpr (CERT) es = fma(cert_norm1(z), ex[u], es);
+    if constexpr (CERT) es = fma(tree_abs(z), ex[u], es);
   };
   (((Ps < k1) ? (term(row_bcast<(2 * Ps) % 16>(Ps < 8 ? c : c2), 2 * Ps),
                  term(row_bcast<(2 * Ps + 1) % 16>(Ps < 8 ? c : c2), 2 * Ps + 1), 0)
@@ -1045,8 +1060,8 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
         dd_mac<CERT>(s.re, dd_neg(x.im), y.im, r);
         dd_mac<CERT>(s.im, x.im, y.re, r);
         if constexpr (CERT) {
-          const double Y = cddc_norm1(y);
-          es = fma(cddc_norm1(x), ey, fma(ex, Y + ey, es + r));
+          const double Y = tree_abs(y);
+          es = fma(tree_abs(x), ey, fma(ex, Y + ey, es + r));
         }
       };
       ChainC pe, po;
@@ -1161,7 +1176,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       p0 = ldc[2 * (yo + d + 1) + half];
       p1v = ldc[2 * (yo + d + 1) + 1 - half];
       if constexpr (CERT) {
-        const double Y = cdd_mag(p0) + cdd_mag(p1v), ey = ldse[yo + d + 1];
+        const double Y = tree_abs(cdd_mag(p0), cdd_mag(p1v)), ey = ldse[yo + d + 1];
         yp = ey;
         yq = Y + ey;
       }
@@ -1186,7 +1201,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       p0 = n0;
       p1v = n1;
       if constexpr (CERT) {
-        const double X = cdd_mag(xr) + cdd_mag(xi), Y = cdd_mag(n0) + cdd_mag(n1);
+        const double X = tree_abs(cdd_mag(xr), cdd_mag(xi)), Y = tree_abs(cdd_mag(n0), cdd_mag(n1));
         a1.e = fma(X, yp, fma(ex, yq, a1.e));
         yp = ey;
         yq = Y + ey;
@@ -1197,7 +1212,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       const dd xr = dd_signed(x0, sx), xi = dd_signed(x1, sx * sgi);
       dd_mac<CERT>(a1.v, xr, p0, a1.r);
       dd_mac<CERT>(a1.v, xi, p1v, a1.r);
-      if constexpr (CERT) a1.e = fma(cdd_mag(xr) + cdd_mag(xi), yp, fma(xe, yq, a1.e));
+      if constexpr (CERT) a1.e = fma(tree_abs(cdd_mag(xr), cdd_mag(xi)), yp, fma(xe, yq, a1.e));
     }
   };
   using Yes = std::true_type;
@@ -1205,7 +1220,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
   // closes a chain: its errors in both components join the bound
   auto close = [&](Acc& a) __attribute__((always_inline)) -> dd {
     const dd v = chain_value<CERT>(a.v, a.r);
-    if constexpr (CERT) a.e += a.r + swap_pair_d(a.r);
+    if constexpr (CERT) a.e += tree_abs(a.r, swap_pair_d(a.r));
     return v;
   };
   auto begin = [](Acc& a, dd v) __attribute__((always_inline)) {
@@ -1214,7 +1229,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
     if constexpr (CERT) a.r = 1e-11 * CERT_U * fabs(v.lo);
   };
   // e + the errors of both components' operations since r was zero
-  auto both = [&](double e, double r) -> double { return CERT ? e + (r + swap_pair_d(r)) : 0.0; };
+  auto both = [&](double e, double r) -> double { return CERT ? e + tree_abs(r, swap_pair_d(r)) : 0.0; };
 #pragma unroll 1
   for (int l = 0; l < T2; ++l) {
     const TreeTask k = tree_table<LOOP, true>.t[l][lane & ~1], kb = tree_table<LOOP, true>.t[l][lane | 1];
@@ -1382,7 +1397,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       if constexpr (CERT) {
         double r;
         coeff = cdd_div_d(s, (double)j, &r);
-        ecoeff = e / (double)j + r + swap_pair_d(r);
+        ecoeff = e / (double)j + tree_abs(r, swap_pair_d(r));
         ldse[eo + j - 1] = ecoeff;
       } else {
         coeff = dd_div_d(s, (double)j);
@@ -1404,7 +1419,7 @@ __global__ __launch_bounds__(64) void haf_tree_dd_kernel(const cplx* __restrict_
       double r;
       const double oe = shfl_xor_d(ecoeff, m);
       coeff = cdd_add(coeff, o, &r);
-      ecoeff = ecoeff + oe + r + swap_pair_d(r);
+      ecoeff = ecoeff + oe + tree_abs(r, swap_pair_d(r));
     } else {
       coeff = dd_add(coeff, o);
     }

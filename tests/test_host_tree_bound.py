@@ -5,6 +5,7 @@ product of the bounds must fail here.
 
 The bound's own arithmetic is in round to nearest; cert_finish inflates the end
 result by 1 + 2 D u for its rounding depth D, here below 64 (7 steps of 5 and the end)."""
+import math
 import shutil
 import subprocess
 from fractions import Fraction
@@ -62,8 +63,12 @@ def add(a, b):
     return a[0] + b[0], a[1] + b[1]
 
 
-def norm(a):
-    return abs(a[0]) + abs(a[1])
+def square(a):
+    return a[0] * a[0] + a[1] * a[1]
+
+
+def norm(a):  # |a| from above
+    return Fraction(math.sqrt(square(a))) * (1 + 4 * U)
 
 
 @pytest.fixture(scope="module")
@@ -83,7 +88,7 @@ def rows(tmp_path_factory):
 
 
 def worst_error(c, d):
-    """Largest |acc_d - exact| over operands moved by their bounds along one direction
+    """Square of the largest |acc_d - exact| over operands moved by their bounds along one direction
     each (real or imaginary, either sign)."""
     best = Fraction(0)
     for sx in ((1, 0), (-1, 0), (0, 1), (0, -1)):
@@ -92,14 +97,14 @@ def worst_error(c, d):
             for i in range(d + 1):
                 a, b = c[i], c[d - i]
                 s = add(s, mul((a[0] + sx[0] * a[2], a[1] + sx[1] * a[2]), (b[3] + sy[0] * b[5], b[4] + sy[1] * b[5])))
-            best = max(best, norm((s[0] - c[d][6], s[1] - c[d][7])))
+            best = max(best, square((s[0] - c[d][6], s[1] - c[d][7])))
     return best
 
 
 def test_products_are_enclosed(rows):
     for kind, c in rows:
         for d in range(H):
-            assert worst_error(c, d) <= c[d][8] * (1 + 2 * 64 * U), (kind, d)
+            assert worst_error(c, d) <= (c[d][8] * (1 + 2 * 64 * U)) ** 2, (kind, d)
 
 
 def test_a_rule_without_the_product_of_bounds_does_not_enclose(rows):
@@ -112,6 +117,6 @@ def test_a_rule_without_the_product_of_bounds_does_not_enclose(rows):
                 a, b = c[i], c[d - i]
                 acc = add(acc, mul(a[:2], b[3:5]))
                 e += 2 * U * norm(acc) + norm(a[:2]) * b[5] + a[2] * norm(b[3:5])
-            if worst_error(c, d) > e * (1 + 2 * 64 * U):
+            if worst_error(c, d) > (e * (1 + 2 * 64 * U)) ** 2:
                 failed.add(kind)
     assert 2 in failed
