@@ -216,15 +216,37 @@ def _rewrite_constant(path: Path, name: str, value: int, out: Path | None = None
     (out or path).write_text(new)
 
 
+TOR_TREE_MODES = 6   # from here on one kernel serves both walks (csrc/tor_tree.hpp)
+TOR_BFS_ALL = 32     # every mode count
+
+
+def choose_tor(times: dict[int, dict[str, float]], margin: float) -> tuple[int, int]:
+    """(grouped_max, bfs_max) from each mode count's times. bfs_max: the largest count up
+    to which breadth-first is never slower than (1 + margin) x depth-first, of the
+    counts that have both walks; every count if it is so at all of them."""
+    bfs_max, grouped_max, still = 0, 0, True
+    for nm in sorted(times):
+        t = times[nm]
+        walk = t["bfs"]
+        if nm < TOR_TREE_MODES:
+            walk = min(walk, t["dfs"])
+            still = still and t["bfs"] <= (1.0 + margin) * t["dfs"]
+            if still:
+                bfs_max = nm
+        if nm <= 10 and t["grouped"] < (1.0 - margin) * walk and grouped_max == nm - 2:
+            grouped_max = nm
+    return grouped_max, (TOR_BFS_ALL if still else bfs_max)
+
+
 def tune_tor(L, torch, reps: int, margin: float, allow_split_change: bool, write, sizes=None) -> None:
     """Breadth-first vs depth-first middle walk per family and mode count (4096
-    physical instances, fewer at 16+ modes); bfs_max = the largest mode count
-    up to which breadth-first is never slower than (1 + margin) x depth-first.
-    The grouped kernel is timed beside them and adopted only with
-    allow_split_change (it changes the split)."""
+    physical instances, fewer at 16+ modes) where both exist, the one kernel of
+    the larger counts beside them; the choice is choose_tor's. The grouped kernel
+    is timed as well and adopted only with allow_split_change (it changes the
+    split)."""
     import ctypes
     from .workloads import threshold_O
-    sizes = sizes or [4, 6, 8, 10, 12, 14, 16, 18, 20]
+    sizes = sizes or [3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20]
     saved = []
     for fam in (0, 1):
         g, b = ctypes.c_int(), ctypes.c_int()
@@ -235,24 +257,21 @@ def tune_tor(L, torch, reps: int, margin: float, allow_split_change: bool, write
     print("|---|---|---|---|---|---|")
     try:
         for fam, tier in ((0, 0), (1, 1)):
-            bfs_max, grouped_max, still = 0, 0, True
+            times = {}
             for nm in sizes:
                 B = 4096 if nm <= 12 else (1024 if nm <= 16 else 256)
                 rng = np.random.default_rng(900 + nm)
                 O = np.stack([threshold_O(nm, rng) for _ in range(B)]).astype(np.complex128)
                 go, stream = _device_call(L, torch, 3, tier, O)
-                t = {}
-                for label, gm, bm in (("dfs", 0, 0), ("bfs", 0, 32), ("grouped", 10, 32)):
+                t = times[nm] = {}
+                for label, gm, bm in (("dfs", 0, 0), ("bfs", 0, TOR_BFS_ALL), ("grouped", 10, TOR_BFS_ALL)):
+                    if label == "dfs" and nm >= TOR_TREE_MODES:
+                        continue
                     L.gbs_tor_set_schedule(fam, gm, bm)
                     t[label] = _median_ms(torch, stream, go, reps)
-                print(f"| {FAMILIES[fam][0]} | {nm} | {B} | {t['dfs']:.3f} | {t['bfs']:.3f} | {t['grouped']:.3f} |",
-                      flush=True)
-                if still and t["bfs"] <= (1.0 + margin) * t["dfs"]:
-                    bfs_max = nm
-                else:
-                    still = False
-                if nm <= 10 and t["grouped"] < (1.0 - margin) * min(t["bfs"], t["dfs"]) and grouped_max == nm - 2:
-                    grouped_max = nm
+                dfs = f"{t['dfs']:.3f}" if "dfs" in t else "-"
+                print(f"| {FAMILIES[fam][0]} | {nm} | {B} | {dfs} | {t['bfs']:.3f} | {t['grouped']:.3f} |", flush=True)
+            grouped_max, bfs_max = choose_tor(times, margin)
             chosen[fam] = (grouped_max if allow_split_change else saved[fam][0], bfs_max)
     finally:
         for fam, (g, b) in enumerate(saved):
