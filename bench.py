@@ -52,15 +52,15 @@ TRAFFIC_N24 = 13742848
 EXECUTED_F64 = {
     "perm_fp64_n24": (2.014479e+09, 1.888513e+07),
     "perm_fp64_n16": (5169792, 48586),
-    "haf_fp64_n16": (7939584, 65744),
-    "haf_fp64_n24": (5.18053e+08, 4206890),
-    "lhaf_fp64_n16": (9162176, 78319),
-    "lhaf_fp64_n24": (5.749229e+08, 4794570),
+    "haf_fp64_n16": (4169856, 35778),
+    "haf_fp64_n24": (1.695419e+08, 1402884),
+    "lhaf_fp64_n16": (4811584, 41965),
+    "lhaf_fp64_n24": (1.880719e+08, 1575679),
     "haf_fp64_config1_n8": (19136, 184.0),
-    "tor_fp64_nm8": (60288, 611),
-    "tor_fp64_nm12": (505728, 5099),
-    "tor_fp64_nm16": (8459776, 85258),
-    "tor_fp64_nm20": (1.429188e+08, 1441431),
+    "tor_fp64_nm8": (40896, 408),
+    "tor_fp64_nm12": (377792, 3712),
+    "tor_fp64_nm16": (6787712, 67034),
+    "tor_fp64_nm20": (1.219794e+08, 1209864),
 }
 # FP64 VALU wave instructions per second at the 78.6 TFLOP/s peak: one per CU
 # per clock (256 CUs, 2.4 GHz; an FMA over 64 lanes is 128 flop)
