@@ -1365,11 +1365,14 @@ static void launch_phase(const HafJob* jobs, int njobs, typename Ar::T* const* p
 }
 
 // Series tree of one bucket of side N = 2 H >= TREE_MIN_N: one workgroup per
-// instance and leading-pair pattern, partials [B][tree_parts(N)]. The line lies at
-// N = 14 because the power-trace kernels of N <= 12 are fused in one launch whose
-// values its own tests pin; at N = 14 (B = 4000) the tree took 249 us where the
-// per-size launches took 552 (loop 317 / 639, certified 492 / 851, dd B = 512
-// 327 / 741), at N = 24 (B = 256) 1.40 ms for 4.02, and it leads at every larger side.
+// instance and leading-pair pattern, partials [B][tree_parts(N)]. At N = 14 (B = 4000)
+// the tree took 249 us where the per-size launches took 552 (loop 317 / 639, certified
+// 492 / 851, dd B = 2048 1366 / 2248), at N = 24 (B = 256) 1.40 ms for 4.02, and it leads at
+// every larger side. The line lies at N = 14 although the tree, built down to side 10,
+// was faster there too on complex matrices (B = 4096, kernels of N <= 12 / tree: N = 10
+// 50 / 39 us, N = 12 117 / 86, loop 166 / 131, dd 751 / 719, certified dd N = 10 1103 / 398):
+// below it values are pinned bit for bit to the per-size launches, also those of the
+// fused kernel, which runs real matrices in real arithmetic, and would change.
 template <class Ar, bool LOOP, int MODE, int H>
 static void launch_tree_h(const HafJob& j, typename Ar::T* part, double* part_abs, hipStream_t st) {
   const dim3 grid((unsigned)j.B * (unsigned)tree_parts(2 * H)), wg(64);
