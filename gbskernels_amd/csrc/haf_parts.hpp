@@ -35,12 +35,16 @@ constexpr int haf_nchunks(int n, int S) {
   return (c + ch - 1) / ch;
 }
 // partial slots per instance (all phases) and the first slot of phase S
+constexpr int haf_nparts(int n) {
+  int t = 0;
+  for (int m = 1; m <= n; ++m) t += haf_nchunks(n, 2 * m);
+  return t;
+}
 constexpr int haf_part_offset(int n, int S) {
   int t = 0;
   for (int m = 1; m < S / 2; ++m) t += haf_nchunks(n, 2 * m);
   return t;
 }
-constexpr int haf_nparts(int n) { return haf_part_offset(n, 2 * n + 2); }
 
 // partials of one instance of side N (even, 2 .. TREE_MAX_N)
 constexpr int haf_parts(int N) { return N > HAF_PHASE_MAX_N ? tree_parts(N) : haf_nparts(N / 2); }
