@@ -1486,7 +1486,10 @@ static void launch_tor_rt(int nm, int T1, const cplx* d_in, int B, typename Ar::
     // shorter trailing walks keep ten leading modes)
     constexpr int LB = TOR_BATCH_MAX_MODES - TOR_T2 - Ar::RMAX, LX = TOR_MAX_MODES - TOR_T2 - R;
     constexpr int LM = LB > 10 ? LB : 10;
-    if (T1 <= LM) {
+    if (tor_lead_lds<Ar, LM>() && T1 == 0) {  // no LDS for leading modes
+      hipLaunchKernelGGL((tor_tree_kernel<Ar, R, KAPPA, tor_lead_lds<Ar, LM>() ? 0 : LM>), grid, dim3(64), 0, st, d_in,
+                         T1, part, part_abs, dir);
+    } else if (T1 <= LM) {
       hipLaunchKernelGGL((tor_tree_kernel<Ar, R, KAPPA, LM>), grid, dim3(64), 0, st, d_in, T1, part, part_abs, dir);
     } else if constexpr (R == Ar::RMAX && !KAPPA) {
       hipLaunchKernelGGL((tor_tree_kernel<Ar, R, KAPPA, LX>), grid, dim3(64), 0, st, d_in, T1, part, part_abs, dir);

@@ -110,6 +110,27 @@ __device__ __forceinline__ void lane_include(const T* N, T* Y, bool inc, bool& b
 template <class Ar>
 constexpr int tor_tree_waves() { return std::is_same<Ar, RF64>::value || std::is_same<Ar, RDD>::value ? 2 : 1; }
 
+// t_k = read(k) for k < N, a barrier, then write(k, t_k): no array (it went to scratch)
+template <int N, class Rd, class Wr>
+__device__ __forceinline__ void read_then_write(const Rd& read, const Wr& write) {
+  const auto t = read(N - 1);
+  if constexpr (N > 1)
+    read_then_write<N - 1>(read, write);
+  else
+    __syncthreads();
+  write(N - 1, t);
+}
+
+// Certified dd keeps up to 11 leading modes in LDS, one entry of the active block a
+// lane and step (eliminate, tor.hip): a step of its arithmetic is some 100 operations,
+// and one column a lane leaves 64 - D lanes idle, 2.8 times the steps at 10 leading
+// modes and no trailing ones. General workgroup / one column a lane / this, us: one instance
+// over the device at 12 / 16 / 18 modes 83 / 102 / 83, 126 / 155 / 125, 169 / 192 / 161, one of a batch at
+// 18 modes 149 / 169 / 136, B = 4096 at 12 / 16 modes 4235 / 3493 / 2993, 78300 / 66100 / 53700. Without
+// leading modes LM is 0 (their LDS cost a third of the waves: 8 modes, B = 1024 48 -> 60 us).
+template <class Ar, int LM>
+constexpr bool tor_lead_lds() { return std::is_same<Ar, RCDD>::value && LM > 0 && LM <= 11; }
+
 // LM: leading modes the register columns have room for.
 template <class Ar, int R, bool KAPPA, int LM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tor_tree_waves<Ar>()))) void tor_tree_kernel(
@@ -120,7 +141,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tor_tree_wav
   constexpr int BASE = TOR_T2 + R, DB = 2 * BASE;
   constexpr int LV = TREE_LDS_LEVELS, MT = BASE - LV;  // MT modes left where the lanes take over
   static_assert(TOR_T2 == LV + 2 && DB + 2 * LM <= 64, "two middle modes in registers, one column a lane");
-  __shared__ T lev[tree_region_at(BASE, LV + 1)];
+  constexpr bool LEAD_LDS = tor_lead_lds<Ar, LM>();
+  constexpr int LEVN = tree_region_at(BASE, LV + 1), WN = LEAD_LDS ? (DB + 2 * LM) * (DB + 2 * LM) : 0;
+  __shared__ T lev[LEVN > WN ? LEVN : WN];
   __shared__ T bdet[(2 << LV) - 1];  // determinants, level d node n at 2^d - 1 + n
   __shared__ unsigned short bij[(BASE * (BASE - 1)) / 2];
   const int lane = threadIdx.x;
@@ -138,81 +161,125 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tor_tree_wav
   // included leading ones), mode-major: lane c holds column c, X[r] row r. Only
   // active entries are read; the workgroup with every leading mode included
   // reads all of O, so a complex entry anywhere still flags the instance.
-  T X[DB + 2 * LM];
   bool bad = false;
-  {
+  T det = Ar::one();
+  if constexpr (LEAD_LDS) {
+    // W: the active block, row-major, included leading modes first
+    __shared__ unsigned char amode[BASE + LM];
+    T* const W = lev;
     const cplx* O = mats + b * dim * dim;
-    int mc = T1 + (lane >> 1);
-    if (lane >= DB) {
-      mc = 0;
+    const int D = DB + 2 * k1;
+    if (lane < BASE + k1) {
       unsigned rest = p1;
-      const int q = (lane - DB) >> 1;
-      for (int i = 0; i < q; ++i) rest &= rest - 1;
-      if (rest) mc = __builtin_ctz(rest);
+      for (int i = 0; i < lane && rest; ++i) rest &= rest - 1;
+      amode[lane] = (unsigned char)(lane < k1 ? __builtin_ctz(rest) : T1 + lane - k1);
     }
-    const bool on = lane < DB + 2 * k1;
-    const int gc = on ? mc + (lane & 1) * nm : 0;
-    cplx raw[DB + 2 * LM];
+    __syncthreads();
+    for (int e = lane; e < D * D; e += 64) {
+      const int r = e / D, c = e - r * D;
+      const cplx o = O[(amode[r >> 1] + (r & 1) * nm) * dim + amode[c >> 1] + (c & 1) * nm];
+      W[e] = r == c ? Ar::one_minus(o) : Ar::neg(o);
+      bad |= !Ar::domain(o);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int q = 0; q < k1; ++q) {
+      const T a = eliminate<Ar>(W, D, 2 * q);
+      const T c = eliminate<Ar>(W, D, 2 * q + 1);
+      bad |= !Ar::pos(a) || !Ar::pos(c);
+      det = Ar::mul(det, Ar::mul(a, c));
+    }
+    // level 0 in place: read everything, then write
+    constexpr int N0 = DB * (DB + 1) / 2, PER = (N0 + 63) / 64;
+    read_then_write<PER>(
+        [&](int k) __attribute__((always_inline)) {
+          int i = 0, j = 0;
+          if (lane + 64 * k < N0) tri_decode(lane + 64 * k, i, j);
+          return W[(2 * k1 + i) * D + 2 * k1 + j];
+        },
+        [&](int k, const T& t) __attribute__((always_inline)) {
+          if (lane + 64 * k < N0) {
+            int i, j;
+            tri_decode(lane + 64 * k, i, j);
+            const int I = BASE - 1 - (j >> 1);
+            lev[2 * I * (I + 1) + 2 * (j & 1) + 4 * (BASE - 1 - (i >> 1)) + (i & 1)] = t;
+          }
+        });
+  } else {
+    T X[DB + 2 * LM];
+    {
+      const cplx* O = mats + b * dim * dim;
+      int mc = T1 + (lane >> 1);
+      if (lane >= DB) {
+        mc = 0;
+        unsigned rest = p1;
+        const int q = (lane - DB) >> 1;
+        for (int i = 0; i < q; ++i) rest &= rest - 1;
+        if (rest) mc = __builtin_ctz(rest);
+      }
+      const bool on = lane < DB + 2 * k1;
+      const int gc = on ? mc + (lane & 1) * nm : 0;
+      cplx raw[DB + 2 * LM];
 #pragma unroll
-    for (int r = 0; r < DB; ++r) raw[r] = O[(T1 + (r >> 1) + (r & 1) * nm) * dim + gc];
-    unsigned rest = p1;
+      for (int r = 0; r < DB; ++r) raw[r] = O[(T1 + (r >> 1) + (r & 1) * nm) * dim + gc];
+      unsigned rest = p1;
 #pragma unroll
-    for (int q = 0; q < LM; ++q) {
-      raw[DB + 2 * q] = raw[DB + 2 * q + 1] = cplx{0.0, 0.0};
-      if (q < k1) {
-        const int m = __builtin_ctz(rest);
-        rest &= rest - 1;
-        raw[DB + 2 * q] = O[m * dim + gc];
-        raw[DB + 2 * q + 1] = O[(m + nm) * dim + gc];
+      for (int q = 0; q < LM; ++q) {
+        raw[DB + 2 * q] = raw[DB + 2 * q + 1] = cplx{0.0, 0.0};
+        if (q < k1) {
+          const int m = __builtin_ctz(rest);
+          rest &= rest - 1;
+          raw[DB + 2 * q] = O[m * dim + gc];
+          raw[DB + 2 * q + 1] = O[(m + nm) * dim + gc];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < DB + 2 * LM; ++r) {
+        X[r] = r == lane ? Ar::one_minus(raw[r]) : Ar::neg(raw[r]);
+        bad |= on && !Ar::domain(raw[r]);
       }
     }
-#pragma unroll
-    for (int r = 0; r < DB + 2 * LM; ++r) {
-      X[r] = r == lane ? Ar::one_minus(raw[r]) : Ar::neg(raw[r]);
-      bad |= on && !Ar::domain(raw[r]);
-    }
-  }
 
-  // ---- eliminate the included leading modes (mode order, x then p pivot): the
-  // pivot mode's rows are X[DB], X[DB + 1]; the rows above move down after it
-  T det = Ar::one();
+    // ---- eliminate the included leading modes (mode order, x then p pivot): the
+    // pivot mode's rows are X[DB], X[DB + 1]; the rows above move down after it
 #pragma unroll 1
-  for (int q = 0; q < k1; ++q) {
-    T piv[2];
+    for (int q = 0; q < k1; ++q) {
+      T piv[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int src = DB + 2 * q + t;
-      piv[t] = lane_bcast(X[DB + t], src);
-      const T rp = Ar::recip(piv[t]);
-      auto step = [&](int r) __attribute__((always_inline)) {
-        X[r] = Ar::fms(lane_bcast(Ar::mul(X[r], rp), src), X[DB + t], X[r]);
-      };
+      for (int t = 0; t < 2; ++t) {
+        const int src = DB + 2 * q + t;
+        piv[t] = lane_bcast(X[DB + t], src);
+        const T rp = Ar::recip(piv[t]);
+        auto step = [&](int r) __attribute__((always_inline)) {
+          X[r] = Ar::fms(lane_bcast(Ar::mul(X[r], rp), src), X[DB + t], X[r]);
+        };
 #pragma unroll
-      for (int r = 0; r < DB; ++r) step(r);
-      if (t == 0) step(DB + 1);
+        for (int r = 0; r < DB; ++r) step(r);
+        if (t == 0) step(DB + 1);
 #pragma unroll
-      for (int i = 1; i < LM; ++i)
-        if (q + i < k1) {
-          step(DB + 2 * i);
-          step(DB + 2 * i + 1);
-        }
+        for (int i = 1; i < LM; ++i)
+          if (q + i < k1) {
+            step(DB + 2 * i);
+            step(DB + 2 * i + 1);
+          }
+      }
+      bad |= !Ar::pos(piv[0]) || !Ar::pos(piv[1]);
+      det = Ar::mul(det, Ar::mul(piv[0], piv[1]));
+#pragma unroll
+      for (int r = DB; r + 2 < DB + 2 * LM; ++r) X[r] = X[r + 2];
     }
-    bad |= !Ar::pos(piv[0]) || !Ar::pos(piv[1]);
-    det = Ar::mul(det, Ar::mul(piv[0], piv[1]));
+    // level 0: the lower triangle (row r >= column = lane) in reversed blocks
+    {
+      const int I = BASE - 1 - (lane >> 1);
+      T* const row = lev + 2 * I * (I + 1) + 2 * (lane & 1);
+      if (lane < DB) {
 #pragma unroll
-    for (int r = DB; r + 2 < DB + 2 * LM; ++r) X[r] = X[r + 2];
-  }
-  // level 0: the lower triangle (row r >= column = lane) in reversed blocks
-  {
-    const int I = BASE - 1 - (lane >> 1);
-    T* const row = lev + 2 * I * (I + 1) + 2 * (lane & 1);
-    if (lane < DB) {
-#pragma unroll
-      for (int r = 0; r < DB; ++r)
-        if (r >= lane) row[4 * (BASE - 1 - (r >> 1)) + (r & 1)] = X[r];
+        for (int r = 0; r < DB; ++r)
+          if (r >= lane) row[4 * (BASE - 1 - (r >> 1)) + (r & 1)] = X[r];
+      }
     }
-    if (lane == 0) bdet[0] = det;
   }
+  if (lane == 0) bdet[0] = det;
   __syncthreads();
 
   // ---- middle modes 0..3: node n of level d (pattern bits, first mode most
