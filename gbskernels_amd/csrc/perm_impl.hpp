@@ -178,15 +178,18 @@ __device__ inline void glynn_range_fp64(const cplx* __restrict__ AT,  // LDS, AT
 struct RowSplit {
   int k;  // exponent; INT_MIN: nothing to split (zero, infinite or NaN row)
   __device__ static RowSplit of(double sum) {
-    return RowSplit{sum > 0.0 && sum < INFINITY ? ilogb(fmin(sum * (1.0 + 0x1p-40), 1.79769313486231570e308)) + 1 : INT_MIN};
+    // frexp's exponent: 2^k > sum (one instruction, subnormal numbers too)
+    return RowSplit{sum > 0.0 && sum < INFINITY
+                        ? __builtin_amdgcn_frexp_exp(fmin(sum * (1.0 + 0x1p-40), 1.79769313486231570e308))
+                        : INT_MIN};
   }
   __device__ double hi(double a) const { return k == INT_MIN ? a : ldexp(rint(ldexp(a, 53 - k)), k - 53); }
 };
 
-// split the MPW staged matrices in place: AT keeps the high parts, AL gets the low
+// split the `mats` staged matrices in place: AT keeps the high parts, AL gets the low
 template <int N, int MPW>
-__device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N]) {
-  for (int t = threadIdx.x; t < MPW * N * 2; t += 64) {  // (matrix, row, component)
+__device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N], int mats) {
+  for (int t = threadIdx.x; t < mats * N * 2; t += 64) {  // (matrix, row, component)
     const int q = t / (2 * N), r = (t >> 1) % N;
     double* const a = reinterpret_cast<double*>(&AT[q][r]) + (t & 1);
     double* const l = reinterpret_cast<double*>(&AL[q][r]) + (t & 1);
@@ -204,8 +207,47 @@ __device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N]
   __syncthreads();
 }
 
+// Up to this side a lane splits its own copy of the matrix in registers and its few
+// terms are unrolled (2^M is 2^MLIM there whatever the table says): the pass over
+// LDS and its barrier took longer than the additions it saves. dd, B = 200000: n = 2 / 3 / 4
+// 5.0 / 12.5 / 28.5 us with double-double additions, 6.2 / 15.1 / 34.9 split in LDS, 5.3 / 10.6 / 23.0 here.
+constexpr int PERM_DD_REG = 4;
+template <int N>
+__device__ __forceinline__ void split_own(const cplx* A, cplx (&H)[N * N], cplx (&L)[N * N]) {
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      H[c * N + r] = A[c * N + r];
+      sr += fabs(H[c * N + r].re);
+      si += fabs(H[c * N + r].im);
+    }
+    const RowSplit kr = RowSplit::of(sr), ki = RowSplit::of(si);
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      const cplx a = H[c * N + r], h{kr.hi(a.re), ki.hi(a.im)};
+      H[c * N + r] = h;
+      L[c * N + r] = cplx{kr.k == INT_MIN ? 0.0 : a.re - h.re, ki.k == INT_MIN ? 0.0 : a.im - h.im};
+    }
+  }
+}
+
 // one row's sum as a normalised double-double
 __device__ inline ddc row_sum(cplx h, cplx l) { return ddc{fast_two_sum(h.re, l.re), fast_two_sum(h.im, l.im)}; }
+
+// f(b), ..., f(e - 1); small sides: f(b) .. f(E - 1) unrolled (e == E there)
+template <int N, int E, class F>
+__device__ __forceinline__ void perm_dd_loop(int b, int e, const F& f) {
+  if constexpr (N <= PERM_DD_REG) {
+    static_assert(PermCfg<N, 1>::MLIM <= 2, "no entry below 2^2 terms a lane: M is MLIM");
+#pragma unroll
+    for (int j = 1; j < E; ++j) f(j);
+  } else {
+#pragma unroll 1
+    for (int j = b; j < e; ++j) f(j);
+  }
+}
 
 // Same walk in complex double-double (reference: core/permanent_dd.cu:34-73,
 // cpu_ref/permanent.py:142-189). What bounds it: FP64 issue, 842 operations
@@ -214,8 +256,7 @@ __device__ inline ddc row_sum(cplx h, cplx l) { return ddc{fast_two_sum(h.re, l.
 // 16 / 20 (B = 16384 / 16384 / 16384 / 238) 66 / 1066 / 18381 / 5501 -> 47 / 805 / 14159 /
 // 4086 us, certified n = 16 (B = 1907) 5549 -> 3139 us; values the same binary64 bits.
 template <int N>
-__device__ inline void glynn_range_dd(const cplx* __restrict__ AT, const cplx* __restrict__ AL, uint32_t start, int M,
-                                      ddc& acc_out) {
+__device__ __forceinline__ void glynn_range_dd(const cplx* AT, const cplx* AL, uint32_t start, int M, ddc& acc_out) {
   cplx rh[N], rl[N];
   const uint32_t g = start ^ (start >> 1);
 #pragma unroll
@@ -230,8 +271,8 @@ __device__ inline void glynn_range_dd(const cplx* __restrict__ AT, const cplx* _
       rl[r] = c_axpy(s, AL[c * N + r], rl[r]);
     }
   };
-#pragma unroll 1
-  for (int c = 1; c < N; ++c) update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c);
+  auto first = [&](int c) __attribute__((always_inline)) { update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c); };
+  perm_dd_loop<N, N>(1, N, first);
   auto product = [&]() {
     // two interleaved chains (even / odd rows), then their product
     ddc t0 = row_sum(rh[0], rl[0]);
@@ -244,14 +285,14 @@ __device__ inline void glynn_range_dd(const cplx* __restrict__ AT, const cplx* _
     return ddc_mul(t0, t1);
   };
   ddc acc = product();
-  const uint32_t nsteps = 1u << M;
-  for (uint32_t j = 1; j < nsteps; ++j) {
+  auto term = [&](int j) __attribute__((always_inline)) {
     const int k = __builtin_ctz(j);
-    const uint32_t i = start + j;
+    const uint32_t i = start + (uint32_t)j;
     update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     ddc p = product();
-    acc = (j & 1u) ? ddc_sub(acc, p) : ddc_add(acc, p);
-  }
+    acc = (j & 1) ? ddc_sub(acc, p) : ddc_add(acc, p);
+  };
+  perm_dd_loop<N, 1 << PermCfg<N, 1>::MLIM>(1, 1 << M, term);
   acc_out = acc;
 }
 
@@ -269,8 +310,8 @@ __device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
 // the signed accumulation propagate it with the 1-norm product rule plus each
 // operation's own error.
 template <int N>
-__device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, const cplx* __restrict__ AL, uint32_t start,
-                                          int M, ddc& acc_out, double& e_out) {
+__device__ __forceinline__ void glynn_range_ddcert(const cplx* AT, const cplx* AL, uint32_t start, int M, ddc& acc_out,
+                                                   double& e_out) {
   cplx rh[N], rl[N];
   const uint32_t g = start ^ (start >> 1);
   double E = 0.0;
@@ -290,8 +331,8 @@ __device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, const cpl
     }
     E += fma(CERT_U, m, CERT_UFL);
   };
-#pragma unroll 1
-  for (int c = 1; c < N; ++c) update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c);
+  auto first = [&](int c) __attribute__((always_inline)) { update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c); };
+  perm_dd_loop<N, N>(1, N, first);
   auto product = [&](double& ep) {
     ddc t0 = row_sum(rh[0], rl[0]);
     double e0 = E;
@@ -326,16 +367,16 @@ __device__ inline void glynn_range_ddcert(const cplx* __restrict__ AT, const cpl
   };
   double ea;
   ddc acc = product(ea);
-  const uint32_t nsteps = 1u << M;
-  for (uint32_t j = 1; j < nsteps; ++j) {
+  auto term = [&](int j) __attribute__((always_inline)) {
     const int k = __builtin_ctz(j);
-    const uint32_t i = start + j;
+    const uint32_t i = start + (uint32_t)j;
     update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     double ep, eo;
     const ddc p = product(ep);
-    acc = (j & 1u) ? cddc_sub(acc, p, &eo) : cddc_add(acc, p, &eo);
+    acc = (j & 1) ? cddc_sub(acc, p, &eo) : cddc_add(acc, p, &eo);
     ea = ea + ep + eo;
-  }
+  };
+  perm_dd_loop<N, 1 << PermCfg<N, 1>::MLIM>(1, 1 << M, term);
   acc_out = acc;
   e_out = ea;
 }
@@ -380,7 +421,7 @@ constexpr int perm_min_waves() { return (MODE == PERM_CERT || MODE == PERM_DDCER
 // complex numbers of LDS one workgroup uses: the matrices (dd: high, then low parts)
 template <int N, int MODE>
 constexpr int perm_lds() {
-  return (64 / PermCfg<N, perm_is_dd(MODE) ? 1 : 0>::LPM) * N * N * (perm_is_dd(MODE) ? 2 : 1);
+  return (64 / PermCfg<N, perm_is_dd(MODE) ? 1 : 0>::LPM) * N * N * (perm_is_dd(MODE) && N > PERM_DD_REG ? 2 : 1);
 }
 
 template <int N, int MODE>
@@ -412,9 +453,9 @@ __device__ __forceinline__ void perm_workgroup(const cplx* __restrict__ mats, in
   // (eight loads in flight a lane: one at a time cost a round trip each, 8 us of a
   // 29 us call at n = 8 with the matrices in host memory)
   const cplx* const src = mats + mat0 * (N * N);
-  const int have = (int)(B - mat0 < MPW ? B - mat0 : MPW) * (N * N);
+  const int nmat = (int)(B - mat0 < MPW ? B - mat0 : MPW), have = nmat * (N * N);
 #pragma unroll 1
-  for (int e0 = lane; e0 < MPW * N * N; e0 += 64 * 8) {
+  for (int e0 = lane; e0 < have; e0 += 64 * 8) {  // lanes of absent matrices walk what LDS holds, and store nothing
     cplx v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = e0 + 64 * u < have ? src[e0 + 64 * u] : cplx{0.0, 0.0};
@@ -429,16 +470,25 @@ __device__ __forceinline__ void perm_workgroup(const cplx* __restrict__ mats, in
   const uint32_t start = ((uint32_t)chunk * LPM + (uint32_t)sub) << M;
   if constexpr (perm_is_dd(MODE)) {
     constexpr bool DDCERT = MODE == PERM_DDCERT;
-    cplx(&AL)[MPW][N * N] = *reinterpret_cast<cplx(*)[MPW][N * N]>(lds + MPW * N * N);
-    split_rows<N, MPW>(AT, AL);
     ddc acc;
     double ea = 0.0;
-    if constexpr (DDCERT) {
-      glynn_range_ddcert<N>(AT[gidx], AL[gidx], start, M, acc, ea);
-      cddc_group_sum<LPM>(acc, ea);
+    auto walk = [&](const cplx* H, const cplx* L) __attribute__((always_inline)) {
+      if constexpr (DDCERT) {
+        glynn_range_ddcert<N>(H, L, start, M, acc, ea);
+        cddc_group_sum<LPM>(acc, ea);
+      } else {
+        glynn_range_dd<N>(H, L, start, M, acc);
+        acc = group_sum<LPM>(acc);
+      }
+    };
+    if constexpr (N <= PERM_DD_REG) {
+      cplx H[N * N], L[N * N];
+      split_own<N>(AT[gidx], H, L);
+      walk(H, L);
     } else {
-      glynn_range_dd<N>(AT[gidx], AL[gidx], start, M, acc);
-      acc = group_sum<LPM>(acc);
+      cplx(&AL)[MPW][N * N] = *reinterpret_cast<cplx(*)[MPW][N * N]>(lds + MPW * N * N);
+      split_rows<N, MPW>(AT, AL, nmat);
+      walk(AT[gidx], AL[gidx]);
     }
     if (sub == 0 && b < B) {
       if (W == 1) {
