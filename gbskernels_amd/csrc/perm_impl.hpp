@@ -184,19 +184,39 @@ struct RowSplit {
                         : INT_MIN};
   }
   __device__ double hi(double a) const { return k == INT_MIN ? a : ldexp(rint(ldexp(a, 53 - k)), k - 53); }
+  // The low sums do not round either if the smallest nonzero entry, whose frexp
+  // exponent is `least`, is not far below: low parts are multiples of 2^(least - 53)
+  // and n of them, at most 2^(k - 54) each, stay below 2^53 of those (n <= 2^5).
+  __device__ bool exact(int least) const { return k == INT_MIN || k - 49 <= least; }
 };
+// min(least, frexp exponent of a), a nonzero
+__device__ __forceinline__ int min_exp(double a, int least) {
+  const int e = __builtin_amdgcn_frexp_exp(a);
+  return a != 0.0 && e < least ? e : least;
+}
 
-// split the `mats` staged matrices in place: AT keeps the high parts, AL gets the low
-template <int N, int MPW>
-__device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N], int mats) {
+// split the `mats` staged matrices in place: AT keeps the high parts, AL gets the
+// low; inexact[q] (CERT): a low sum of matrix q may round
+template <int N, int MPW, bool CERT>
+__device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N], int mats, int (&inexact)[MPW]) {
+  static_assert(N <= 32, "RowSplit::exact");
+  if constexpr (CERT) {
+    for (int q = threadIdx.x; q < MPW; q += 64) inexact[q] = 0;
+    __syncthreads();
+  }
   for (int t = threadIdx.x; t < mats * N * 2; t += 64) {  // (matrix, row, component)
     const int q = t / (2 * N), r = (t >> 1) % N;
     double* const a = reinterpret_cast<double*>(&AT[q][r]) + (t & 1);
     double* const l = reinterpret_cast<double*>(&AL[q][r]) + (t & 1);
     double sum = 0.0;
+    int least = INT_MAX;
 #pragma unroll 4
-    for (int c = 0; c < N; ++c) sum += fabs(a[2 * c * N]);
+    for (int c = 0; c < N; ++c) {
+      sum += fabs(a[2 * c * N]);
+      if constexpr (CERT) least = min_exp(a[2 * c * N], least);
+    }
     const RowSplit s = RowSplit::of(sum);
+    if (CERT && !s.exact(least)) inexact[q] = 1;
 #pragma unroll 4
     for (int c = 0; c < N; ++c) {
       const double v = a[2 * c * N], h = s.hi(v);
@@ -213,17 +233,22 @@ __device__ inline void split_rows(cplx (&AT)[MPW][N * N], cplx (&AL)[MPW][N * N]
 // 5.0 / 12.5 / 28.5 us with double-double additions, 6.2 / 15.1 / 34.9 split in LDS, 5.3 / 10.6 / 23.0 here.
 constexpr int PERM_DD_REG = 4;
 template <int N>
-__device__ __forceinline__ void split_own(const cplx* A, cplx (&H)[N * N], cplx (&L)[N * N]) {
+__device__ __forceinline__ bool split_own(const cplx* A, cplx (&H)[N * N], cplx (&L)[N * N]) {
+  bool exact = true;  // no low sum rounds
 #pragma unroll
   for (int r = 0; r < N; ++r) {
     double sr = 0.0, si = 0.0;
+    int lr = INT_MAX, li = INT_MAX;
 #pragma unroll
     for (int c = 0; c < N; ++c) {
       H[c * N + r] = A[c * N + r];
       sr += fabs(H[c * N + r].re);
       si += fabs(H[c * N + r].im);
+      lr = min_exp(H[c * N + r].re, lr);
+      li = min_exp(H[c * N + r].im, li);
     }
     const RowSplit kr = RowSplit::of(sr), ki = RowSplit::of(si);
+    exact = exact && kr.exact(lr) && ki.exact(li);
 #pragma unroll
     for (int c = 0; c < N; ++c) {
       const cplx a = H[c * N + r], h{kr.hi(a.re), ki.hi(a.im)};
@@ -231,21 +256,31 @@ __device__ __forceinline__ void split_own(const cplx* A, cplx (&H)[N * N], cplx 
       L[c * N + r] = cplx{kr.k == INT_MIN ? 0.0 : a.re - h.re, ki.k == INT_MIN ? 0.0 : a.im - h.im};
     }
   }
+  return exact;
 }
 
 // one row's sum as a normalised double-double
 __device__ inline ddc row_sum(cplx h, cplx l) { return ddc{fast_two_sum(h.re, l.re), fast_two_sum(h.im, l.im)}; }
 
-// f(b), ..., f(e - 1); small sides: f(b) .. f(E - 1) unrolled (e == E there)
+// f(1), ..., f(e - 1); small sides unrolled, e = E there
 template <int N, int E, class F>
-__device__ __forceinline__ void perm_dd_loop(int b, int e, const F& f) {
+__device__ __forceinline__ void perm_dd_terms(uint32_t e, const F& f) {
   if constexpr (N <= PERM_DD_REG) {
     static_assert(PermCfg<N, 1>::MLIM <= 2, "no entry below 2^2 terms a lane: M is MLIM");
 #pragma unroll
-    for (int j = 1; j < E; ++j) f(j);
+    for (uint32_t j = 1; j < (uint32_t)E; ++j) f(j);
+  } else {
+    for (uint32_t j = 1; j < e; ++j) f(j);
+  }
+}
+template <int N, class F>
+__device__ __forceinline__ void perm_dd_columns(const F& f) {
+  if constexpr (N <= PERM_DD_REG) {
+#pragma unroll
+    for (int c = 1; c < N; ++c) f(c);
   } else {
 #pragma unroll 1
-    for (int j = b; j < e; ++j) f(j);
+    for (int c = 1; c < N; ++c) f(c);
   }
 }
 
@@ -272,7 +307,7 @@ __device__ __forceinline__ void glynn_range_dd(const cplx* AT, const cplx* AL, u
     }
   };
   auto first = [&](int c) __attribute__((always_inline)) { update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c); };
-  perm_dd_loop<N, N>(1, N, first);
+  perm_dd_columns<N>(first);
   auto product = [&]() {
     // two interleaved chains (even / odd rows), then their product
     ddc t0 = row_sum(rh[0], rl[0]);
@@ -285,14 +320,14 @@ __device__ __forceinline__ void glynn_range_dd(const cplx* AT, const cplx* AL, u
     return ddc_mul(t0, t1);
   };
   ddc acc = product();
-  auto term = [&](int j) __attribute__((always_inline)) {
+  auto term = [&](uint32_t j) __attribute__((always_inline)) {
     const int k = __builtin_ctz(j);
-    const uint32_t i = start + (uint32_t)j;
+    const uint32_t i = start + j;
     update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     ddc p = product();
-    acc = (j & 1) ? ddc_sub(acc, p) : ddc_add(acc, p);
+    acc = (j & 1u) ? ddc_sub(acc, p) : ddc_add(acc, p);
   };
-  perm_dd_loop<N, 1 << PermCfg<N, 1>::MLIM>(1, 1 << M, term);
+  perm_dd_terms<N, 1 << PermCfg<N, 1>::MLIM>(1u << M, term);
   acc_out = acc;
 }
 
@@ -304,16 +339,21 @@ __device__ __forceinline__ void glynn_range_dd(const cplx* AT, const cplx* AL, u
 __device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
 
 // glynn_range_dd with a running bound (certified double-double). The values
-// are glynn_range_dd's bit for bit. E bounds the error of every row sum (high
-// sums are exact; each row receives the same updates, so one bound serves all
-// rows: each step adds the largest of the N low sums' roundings); products and
-// the signed accumulation propagate it with the 1-norm product rule plus each
-// operation's own error.
+// are glynn_range_dd's bit for bit. E bounds the error of every row sum: zero where
+// neither high nor low sums round (exact, RowSplit), which entries within 2^49 of
+// their row's sum ensure; else each step adds the largest of the N low sums'
+// roundings, u |low sum| (so charged for every matrix, bounds of cancelling inputs
+// were 1.9, 2.6 and 9 times as wide as with double-double additions at n = 16, 17 and
+// 22; with rows that span 24 decades they are 1.2, 1.9 and 3.6 times at n = 6, 10 and 22.
+// The errors themselves, by TwoSum, take these away but cost 1.12-1.43 times the time,
+// in a branch of their own 1.15-1.2 times from n = 15 on, in registers). Products and the signed
+// accumulation propagate it with the 1-norm product rule plus each operation's own error.
 template <int N>
-__device__ __forceinline__ void glynn_range_ddcert(const cplx* AT, const cplx* AL, uint32_t start, int M, ddc& acc_out,
-                                                   double& e_out) {
+__device__ __forceinline__ void glynn_range_ddcert(const cplx* AT, const cplx* AL, uint32_t start, int M, bool exact,
+                                                   ddc& acc_out, double& e_out) {
   cplx rh[N], rl[N];
   const uint32_t g = start ^ (start >> 1);
+  const double eu = exact ? 0.0 : CERT_U, ef = exact ? 0.0 : CERT_UFL;
   double E = 0.0;
 #pragma unroll
   for (int r = 0; r < N; ++r) {
@@ -327,12 +367,14 @@ __device__ __forceinline__ void glynn_range_ddcert(const cplx* AT, const cplx* A
       rh[r] = c_axpy(s, AT[c * N + r], rh[r]);
       rl[r] = c_axpy(s, AL[c * N + r], rl[r]);
       m = fmax(m, cert_norm1(rl[r]));
-      pin(m);
+      // every fifth row: the next rows' loads then pass the barrier; at every row
+      // n = 21 / 24 / 26 (B = 256 / 64 / 16) took 22.7 / 51.5 / 60.2 ms, so 19.0 / 43.8 / 49.6
+      if (r % 5 == 4) pin(m);
     }
-    E += fma(CERT_U, m, CERT_UFL);
+    E += fma(eu, m, ef);
   };
   auto first = [&](int c) __attribute__((always_inline)) { update(((g >> (c - 1)) & 1u) ? -1.0 : 1.0, c); };
-  perm_dd_loop<N, N>(1, N, first);
+  perm_dd_columns<N>(first);
   auto product = [&](double& ep) {
     ddc t0 = row_sum(rh[0], rl[0]);
     double e0 = E;
@@ -367,16 +409,16 @@ __device__ __forceinline__ void glynn_range_ddcert(const cplx* AT, const cplx* A
   };
   double ea;
   ddc acc = product(ea);
-  auto term = [&](int j) __attribute__((always_inline)) {
+  auto term = [&](uint32_t j) __attribute__((always_inline)) {
     const int k = __builtin_ctz(j);
-    const uint32_t i = start + (uint32_t)j;
+    const uint32_t i = start + j;
     update(((i >> (k + 1)) & 1u) ? 2.0 : -2.0, k + 1);
     double ep, eo;
     const ddc p = product(ep);
-    acc = (j & 1) ? cddc_sub(acc, p, &eo) : cddc_add(acc, p, &eo);
+    acc = (j & 1u) ? cddc_sub(acc, p, &eo) : cddc_add(acc, p, &eo);
     ea = ea + ep + eo;
   };
-  perm_dd_loop<N, 1 << PermCfg<N, 1>::MLIM>(1, 1 << M, term);
+  perm_dd_terms<N, 1 << PermCfg<N, 1>::MLIM>(1u << M, term);
   acc_out = acc;
   e_out = ea;
 }
@@ -472,9 +514,9 @@ __device__ __forceinline__ void perm_workgroup(const cplx* __restrict__ mats, in
     constexpr bool DDCERT = MODE == PERM_DDCERT;
     ddc acc;
     double ea = 0.0;
-    auto walk = [&](const cplx* H, const cplx* L) __attribute__((always_inline)) {
+    auto walk = [&](const cplx* H, const cplx* L, bool exact) __attribute__((always_inline)) {
       if constexpr (DDCERT) {
-        glynn_range_ddcert<N>(H, L, start, M, acc, ea);
+        glynn_range_ddcert<N>(H, L, start, M, exact, acc, ea);
         cddc_group_sum<LPM>(acc, ea);
       } else {
         glynn_range_dd<N>(H, L, start, M, acc);
@@ -483,12 +525,21 @@ __device__ __forceinline__ void perm_workgroup(const cplx* __restrict__ mats, in
     };
     if constexpr (N <= PERM_DD_REG) {
       cplx H[N * N], L[N * N];
-      split_own<N>(AT[gidx], H, L);
-      walk(H, L);
+      const bool exact = split_own<N>(AT[gidx], H, L);
+      walk(H, L, exact);
     } else {
       cplx(&AL)[MPW][N * N] = *reinterpret_cast<cplx(*)[MPW][N * N]>(lds + MPW * N * N);
-      split_rows<N, MPW>(AT, AL, nmat);
-      walk(AT[gidx], AL[gidx]);
+      __shared__ int inexact[DDCERT ? MPW : 1];
+      if constexpr (DDCERT) {
+        split_rows<N, MPW, true>(AT, AL, nmat, inexact);
+        int bad = inexact[gidx];
+        if constexpr (LPM == 64) bad = __builtin_amdgcn_readfirstlane(bad);  // one matrix: in scalar registers
+        walk(AT[gidx], AL[gidx], bad == 0);
+      } else {
+        int none[MPW];
+        split_rows<N, MPW, false>(AT, AL, nmat, none);
+        walk(AT[gidx], AL[gidx], true);
+      }
     }
     if (sub == 0 && b < B) {
       if (W == 1) {
